@@ -4,8 +4,8 @@
 //
 // Kernels
 //   fwht_kernel          structured Hadamard rotation, one wavefront per row
-//   append_kernel        rotate -> quantize -> bit-pack (or dequantize), one
-//                        wavefront per (row, stream), packed words written in
+//   append_kernel        rotate -> quantize -> bit-pack (or dequantize), 16
+//                        elements of a row to a lane, packed words written in
 //                        place into the [L, Hkv, capacity, W] slab
 //   unpack_kernel        packed slab -> dense float32 centroid values
 //   decode_kernel<Fmt>   split-K decode attention: each workgroup owns one
@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <mutex>
@@ -103,36 +104,384 @@ __global__ __launch_bounds__(kBlock) void fwht_kernel(const T* __restrict__ x, f
 // ============================================================== append
 
 
-// One wavefront per (row, stream).  Items [0, rows) are keys, [rows, 2 rows)
-// values (when `streams` == 2).  Rows are (l, h, t) in [L, Hkv, seq_new] order.
+// Division of a 32-bit row number by the tokens per group, as a multiply-high
+// and a shift with constants from the host (d >= 1, n < 2^31).
+struct FastDiv {
+  uint32_t mul, shift, d;
+  __device__ uint32_t quot(uint32_t n) const { return (__umulhi(n, mul) + n) >> shift; }
+};
+FastDiv make_fast_div(uint32_t d) {
+  uint32_t s = 0;
+  while ((uint64_t(1) << s) < d) ++s;
+  return {static_cast<uint32_t>(((uint64_t(1) << 32) * ((uint64_t(1) << s) - d)) / d + 1), s, d};
+}
+
+struct AppendArgs {
+  const void* keys;  // [rows, D] per stream, rows (l, h, t) in [L, Hkv, seq_new] order
+  const void* values;
+  uint32_t rows;
+  FastDiv seq_new;
+  int rotate_keys, rotate_values;
+  int wide;  // sources and outputs 16-byte aligned: vector loads and stores
+  const float* signs_left;
+  const float* signs_right;
+  float sqrt_d;
+  const float* key_bnd;
+  const float* value_bnd;
+  const float* key_cent;
+  const float* value_cent;
+  uint32_t* key_codes;
+  uint32_t* value_codes;
+  int64_t capacity, offset;
+  float* key_out;
+  float* value_out;
+  float* key_scales;
+  float* value_scales;
+};
+
+// Neighbouring floats by their order: key(x) counts the floats below x, with
+// both zeros at 0.
+__device__ __forceinline__ int float_key(float x) {
+  const int i = __float_as_int(x);
+  return i >= 0 ? i : INT_MIN - i;
+}
+__device__ __forceinline__ float key_float(int k) { return __int_as_float(k >= 0 ? k : INT_MIN - k); }
+
+// x / sqrt(D) as wave_rotate_signs rounds it.
+template <int D>
+__device__ __forceinline__ float div_sqrt_d(float x, float sqrt_d) {
+  if constexpr (D == 64) return __fmul_rn(x, 0.125f);
+  if constexpr (D == 256) return __fmul_rn(x, 0.0625f);
+  return __fdiv_rn(x, sqrt_d);
+}
+
+// v[i] += pair * (the partner lane's v[i]) for 16 elements, one operation
+// each: the compiler leaves the DPP move and the fma apart.  The two wait
+// states in front are what a DPP read needs after a VALU write.
+template <int CTRL>
+__device__ __forceinline__ void pair_step(float (&v)[16], float pair) {
+#define TQ_PAIR(i, mode) "v_fmac_f32_dpp %" #i ", %" #i ", %16 " mode " row_mask:0xf bank_mask:0xf\n\t"
+#define TQ_PAIRS(mode)                                                                                             \
+  asm("s_nop 1\n\t" TQ_PAIR(0, mode) TQ_PAIR(1, mode) TQ_PAIR(2, mode) TQ_PAIR(3, mode) TQ_PAIR(4, mode)           \
+          TQ_PAIR(5, mode) TQ_PAIR(6, mode) TQ_PAIR(7, mode) TQ_PAIR(8, mode) TQ_PAIR(9, mode) TQ_PAIR(10, mode)   \
+              TQ_PAIR(11, mode) TQ_PAIR(12, mode) TQ_PAIR(13, mode) TQ_PAIR(14, mode) TQ_PAIR(15, mode)            \
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]),            \
+        "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15])       \
+      : "v"(pair))
+  if constexpr (CTRL == kDppXor1) TQ_PAIRS("quad_perm:[1,0,3,2]");
+  if constexpr (CTRL == kDppXor2) TQ_PAIRS("quad_perm:[2,3,0,1]");
+  if constexpr (CTRL == kDppHalfMirror) TQ_PAIRS("row_half_mirror");
+  if constexpr (CTRL == kDppRor8) TQ_PAIRS("row_ror:8");
+#undef TQ_PAIRS
+#undef TQ_PAIR
+}
+
+constexpr int kAppendBuckets = 64;
+// Rows (of both streams) up to which append_few_kernel runs: 16 wavefronts to
+// a CU, all resident at once.
+constexpr int64_t kAppendFewRows = 4096;
+constexpr int kAppendMaxBlocks = 2048;  // 8 wavefronts per SIMD on 256 CUs: one resident wave of workgroups
+
+// Rotate -> quantize -> pack (or dequantize) rows of one stream (grid y: keys,
+// values), D / 16 lanes to a row and 16 elements to a lane.
 // SCALED (per-vector scales): the rotated row x is quantized as x / s with
 // s = sqrt(mean(x^2)) (1 for a zero row); s is stored at the token's slot of
 // the [L, Hkv, capacity] scale slab, or multiplied into the dequantized
 // values.
+//
+// A prompt's append moves 2 D bytes in and D b / 8 out per fp16 row, so the
+// work per element has to stay near 20 VALU operations to keep up with HBM.
+// Layout: a lane holds the elements 8 l .. 8 l + 7 and D / 2 + 8 l .. of its
+// row, l its place among the row's lanes, so a load is 16 contiguous bytes a
+// lane, a chunk's 8 codes are one word at 4 bits, and of the transform's
+// log2(D) steps the first three and the last stay in registers.  The steps in
+// between are one DPP fma each, own + (+-1) other: l = 4..7 sit mirrored (lane
+// 7 - l + 4), which makes the step 4 apart a row_half_mirror, and the upper
+// lane of a pair keeps the negated difference, right - left.  Its sign is the
+// same on both lanes of every later pair and is undone by the second sign
+// multiply, so every value is wave_fwht's up to the sign of a zero, which no
+// code, mean square or centroid depends on.
+// Quantizer: code(x) = #{k : x > b_k}.  The division by sqrt(D) is monotone,
+// so x / sqrt(D) > b is x > T with T the largest float whose quotient does
+// not exceed b: found once per workgroup, it takes the division (11
+// operations at head_dim 128) out of the loop.  Signs other than +-1 take the
+// division per element instead.  The thresholds are looked up through
+// kAppendBuckets affine buckets of x: with at most one threshold to a bucket,
+// code = (thresholds in lower buckets) + (x > the bucket's own), one 8-byte
+// LDS read and 5 operations against 30 for 15 comparisons; a rounded affine
+// map is monotone, so the count is exact for every x.  Codebooks that put two
+// thresholds into one bucket are counted one threshold at a time.
+// Measured: 24 x 8 x 8192 fp16 tokens at head_dim 128, 4-bit (1.0 GB read and
+// written): 230 us, 4.3 TB/s, against 1160 us for a wavefront per row
+// (append_few_kernel); 4 x 8 x 4096 float32 tokens 27 us, 5.5 TB/s (a large
+// device copy reaches 5.1).  fp16 rows are bound by the 15 operations an
+// element, float32 rows by memory.  With per-vector scales the two divisions
+// an element remain (2.1 to 2.8 TB/s for fp16).
 template <int D, int BITS, typename T, bool DEQUANT, bool SCALED>
-__global__ __launch_bounds__(kBlock) void append_kernel(
-    const T* __restrict__ keys, const T* __restrict__ values, int64_t rows, int streams, int64_t seq_new,
-    int rotate_keys, int rotate_values, const float* __restrict__ signs_left, const float* __restrict__ signs_right,
-    float sqrt_d, const float* __restrict__ key_bnd, const float* __restrict__ value_bnd,
-    const float* __restrict__ key_cent, const float* __restrict__ value_cent, uint32_t* __restrict__ key_codes,
-    uint32_t* __restrict__ value_codes, int64_t capacity, int64_t offset, float* __restrict__ key_out,
-    float* __restrict__ value_out, float* __restrict__ key_scales, float* __restrict__ value_scales) {
+__global__ __launch_bounds__(kBlock) void append_kernel(const AppendArgs a) {
+  constexpr int LPR = D / 16;           // lanes per row: 4, 8, 16
+  constexpr int RPW = kWave / LPR;      // rows per wavefront
+  constexpr int RPB = RPW * kWavesPerBlock;
+  constexpr int W = D * BITS / 32;
+  constexpr int NL = (1 << BITS) - 1;   // thresholds
+  constexpr int NB = kAppendBuckets;
+  __shared__ float s_thr[NL];
+  __shared__ int s_at[NL];              // bucket of each threshold
+  __shared__ float2 s_bucket[NB];       // (threshold or +inf, code below it)
+  __shared__ float s_cent[NL + 1];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+  const bool is_v = blockIdx.y != 0;
+  const bool rotate = (is_v ? a.rotate_values : a.rotate_keys) != 0;
+  const float* bnd = is_v ? a.value_bnd : a.key_bnd;
+
+  // this lane's place among its row's lanes
+  const int pl = lane & (LPR - 1);
+  const int l = LPR >= 8 && (pl & 4) ? (pl & 8) + 11 - (pl & 7) : pl;
+  auto dim = [&](int i) { return (i >> 3) * (D / 2) + 8 * l + (i & 7); };  // element i of 16
+  float sg_first[16], sg_second[16];
+  bool unit = true;  // signs are +-1
+  if (rotate) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      sg_first[i] = a.signs_right[dim(i)];
+      sg_second[i] = a.signs_left[dim(i)];
+      unit = unit && fabsf(sg_second[i]) == 1.f;
+      if (__builtin_popcount(l) & 1) sg_second[i] = -sg_second[i];  // an odd number of negated differences
+    }
+  }
+  // Thresholds apply to the undivided transform (`folded`) or to the rotated
+  // value itself.
+  const bool folded = !SCALED && rotate && __syncthreads_and(unit) != 0;
+  if (tid < NL) {
+    const float b = bnd[tid];
+    float t = b == b ? b : INFINITY;  // nothing exceeds a NaN boundary
+    if (folded && fabsf(t) < INFINITY) {
+      int k = float_key(t * a.sqrt_d);
+      while (k < float_key(INFINITY) && div_sqrt_d<D>(key_float(k + 1), a.sqrt_d) <= t) ++k;
+      while (div_sqrt_d<D>(key_float(k), a.sqrt_d) > t) --k;
+      t = key_float(k);
+    }
+    s_thr[tid] = t;
+  }
+  if (DEQUANT && tid <= NL) s_cent[tid] = (is_v ? a.value_cent : a.key_cent)[tid];
+  __syncthreads();
+  float lo = s_thr[0], hi = s_thr[0];
+#pragma unroll
+  for (int k = 1; k < NL; ++k) {
+    lo = fminf(lo, s_thr[k]);
+    hi = fmaxf(hi, s_thr[k]);
+  }
+  // bucket(x): an affine map rounded to an integer by adding 2^23, whose
+  // mantissa then holds it
+  constexpr float kInt = 8388608.f;
+  const float slope = (NB - 2) / (hi - lo), shift = fmaf(-lo, slope, kInt + 1.f);
+  auto bucket = [&](float x) {
+    return __float_as_uint(fminf(fmaxf(fmaf(x, slope, shift), kInt), kInt + (NB - 1))) - 0x4B000000u;
+  };
+  const bool affine = fabsf(slope) < INFINITY && fabsf(shift) < INFINITY;  // uniform
+  if (affine && tid < NL) s_at[tid] = static_cast<int>(bucket(s_thr[tid]));
+  __syncthreads();
+  bool single = affine;  // at most one threshold to a bucket
+  if (affine && tid < NB) {
+    int below = 0, own = 0;
+    float t = INFINITY;
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      below += s_at[k] < tid;
+      own += s_at[k] == tid;
+      if (s_at[k] == tid) t = s_thr[k];
+    }
+    s_bucket[tid] = make_float2(t, __int_as_float(below));
+    single = own <= 1;
+  }
+  const bool lookup = __syncthreads_and(single) != 0;
+
+  const T* src = static_cast<const T*>(is_v ? a.values : a.keys);
+  uint32_t* codes = is_v ? a.value_codes : a.key_codes;
+  float* scales = is_v ? a.value_scales : a.key_scales;
+  float* out = is_v ? a.value_out : a.key_out;
+  // the partner's sign in each step between lanes
+  const float pair1 = (l & 1) ? -1.f : 1.f, pair2 = (l & 2) ? -1.f : 1.f;
+  const float pair4 = (l & 4) ? -1.f : 1.f, pair8 = (l & 8) ? -1.f : 1.f;
+
+  for (uint32_t r0 = blockIdx.x * RPB; r0 < a.rows; r0 += gridDim.x * RPB) {
+    const uint32_t mine = r0 + wave * RPW + lane / LPR;
+    const uint32_t r = min(mine, a.rows - 1);  // lanes past the end repeat the last row and store nothing
+    alignas(16) T e[16];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const T* p = src + static_cast<int64_t>(r) * D + c * (D / 2) + 8 * l;
+      if (a.wide) {
+#pragma unroll
+        for (int q = 0; q < static_cast<int>(sizeof(T) / 2); ++q)
+          reinterpret_cast<uint4*>(e + 8 * c)[q] = reinterpret_cast<const uint4*>(p)[q];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[8 * c + i] = p[i];
+      }
+    }
+    float v[16];
+    if (!rotate) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = to_f32(e[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = fmaf(to_f32(e[i]), sg_first[i], -0.f);  // the product, in one operation from fp16
+#pragma unroll
+      for (int st = 1; st < 8; st <<= 1)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if ((i & st) == 0) {
+            const float x = v[i], y = v[i + st];
+            v[i] = __fadd_rn(x, y);
+            v[i + st] = __fsub_rn(x, y);
+          }
+      pair_step<kDppXor1>(v, pair1);
+      pair_step<kDppXor2>(v, pair2);
+      if constexpr (LPR >= 8) pair_step<kDppHalfMirror>(v, pair4);
+      if constexpr (LPR >= 16) pair_step<kDppRor8>(v, pair8);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float x = v[i], y = v[i + 8];
+        v[i] = __fadd_rn(x, y);
+        v[i + 8] = __fsub_rn(x, y);
+      }
+      if (!folded) {
+        asm volatile("");  // keeps this a branch: the compiler would divide always and select
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = div_sqrt_d<D>(v[i], a.sqrt_d);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = __fmul_rn(v[i], sg_second[i]);
+    }
+    float scale = 1.f;
+    if constexpr (SCALED) {
+      // mean square in the order of a wavefront's lanes holding D / 64
+      // consecutive elements each: a chain over those, then pairs
+      constexpr int E = D / kWave;
+      float ss[16 / E];
+#pragma unroll
+      for (int j = 0; j < 16 / E; ++j) {
+        ss[j] = 0.f;
+#pragma unroll
+        for (int i = 0; i < E; ++i) ss[j] = fmaf(v[j * E + i], v[j * E + i], ss[j]);
+      }
+      constexpr int H = 8 / E;  // partial sums per chunk
+#pragma unroll
+      for (int st = 1; st < H; st <<= 1)
+#pragma unroll
+        for (int j = 0; j < 2 * H; j += 2 * st) ss[j] += ss[j + st];
+      float s0 = ss[0], s1 = ss[H];
+      s0 = group_sum<LPR>(s0);  // pairs, quads, 8 and 16 lanes: l's bits in order
+      s1 = group_sum<LPR>(s1);
+      const float rms = sqrtf((s0 + s1) / static_cast<float>(D));
+      scale = rms > 0.f ? rms : 1.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = v[i] / scale;
+    }
+    uint32_t code[16];
+    if (lookup) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float2 e = s_bucket[bucket(v[i])];
+        code[i] = __float_as_uint(e.y) + (v[i] > e.x ? 1u : 0u);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) code[i] = 0;
+      for (int k = 0; k < NL; ++k) {
+        const float t = s_thr[k];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) code[i] += v[i] > t ? 1u : 0u;
+      }
+    }
+    const bool active = mine < a.rows;
+    if constexpr (DEQUANT) {
+      if (active) {
+        float* row = out + static_cast<int64_t>(r) * D;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          float* p = row + c * (D / 2) + 8 * l;
+          float e[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) e[i] = SCALED ? s_cent[code[8 * c + i]] * scale : s_cent[code[8 * c + i]];
+          if (a.wide) {
+            reinterpret_cast<float4*>(p)[0] = make_float4(e[0], e[1], e[2], e[3]);
+            reinterpret_cast<float4*>(p)[1] = make_float4(e[4], e[5], e[6], e[7]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) p[i] = e[i];
+          }
+        }
+      }
+    } else {
+      uint32_t chunk[2];  // 8 codes: 8 * BITS bits
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        uint32_t w = code[8 * c];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) w |= code[8 * c + i] << (BITS * i);
+        chunk[c] = w;
+      }
+      const uint32_t lh = a.seq_new.quot(r), t = r - lh * a.seq_new.d;
+      const int64_t slot = static_cast<int64_t>(lh) * a.capacity + a.offset + t;
+      uint32_t* dst = codes + slot * W;
+      if constexpr (BITS == 4) {
+        if (active) {
+          dst[l] = chunk[0];
+          dst[W / 2 + l] = chunk[1];
+        }
+      } else {
+        // the chunk of the next place, l + 1: lane + 1, or lane - 1 in the mirrored half
+        auto next = [&](uint32_t x) {
+          const int y = static_cast<int>(x);
+          const int above = __builtin_amdgcn_mov_dpp(y, 0xF9, 0xF, 0xF, true);   // quad_perm [1,2,3,3]
+          if constexpr (LPR < 8) return static_cast<uint32_t>(above);
+          const int below = __builtin_amdgcn_mov_dpp(y, 0x90, 0xF, 0xF, true);   // quad_perm [0,0,1,2]
+          return static_cast<uint32_t>((l & 4) ? below : above);
+        };
+        const uint32_t n0 = next(chunk[0]), n1 = next(chunk[1]);
+        if constexpr (BITS == 3) {
+          // four chunks of 24 bits are three words
+          const int j = l & 3, w = 3 * (l >> 2) + j;
+          if (active && j < 3) {
+            dst[w] = (chunk[0] >> (8 * j)) | (n0 << (24 - 8 * j));
+            dst[W / 2 + w] = (chunk[1] >> (8 * j)) | (n1 << (24 - 8 * j));
+          }
+        } else {
+          if (active && (l & 1) == 0) {
+            dst[l >> 1] = chunk[0] | (n0 << 16);
+            dst[W / 2 + (l >> 1)] = chunk[1] | (n1 << 16);
+          }
+        }
+      }
+      if (SCALED && active && l == 0) scales[slot] = scale;
+    }
+  }
+}
+
+// The same for a few rows (kAppendFewRows): one wavefront per row, D / 64
+// elements to a lane, codes counted one boundary at a time and packed through
+// LDS.  It has no tables to set up: one token x 4 heads at head_dim 256 takes
+// 2.9 us against append_kernel's 4.3, 64 tokens x 8 heads at 64 3.4 against
+// 5.0, but 512 x 8 at 128 5.8 against 5.6 and 1999 x 4 at 64 8.1 against 5.0.
+template <int D, int BITS, typename T, bool DEQUANT, bool SCALED>
+__global__ __launch_bounds__(kBlock) void append_few_kernel(const AppendArgs a) {
   constexpr int E = D / kWave;
   constexpr int W = D * BITS / 32;
   __shared__ uint8_t s_codes[kWavesPerBlock][D];
   const int wave = threadIdx.x >> 6, lane = lane_id();
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + wave;
-  const bool active = item < rows * streams;
-  const bool is_v = item >= rows;
-  const int64_t r = is_v ? item - rows : item;
+  const uint32_t r = blockIdx.x * kWavesPerBlock + wave;
+  const bool active = r < a.rows;
+  const bool is_v = blockIdx.y != 0;
   float scale = 1.f;  // per-vector scale (SCALED)
   if (active) {
-    const T* src = (is_v ? values : keys) + r * D + lane * E;
+    const T* src = static_cast<const T*>(is_v ? a.values : a.keys) + static_cast<int64_t>(r) * D + lane * E;
     float v[E];
 #pragma unroll
     for (int i = 0; i < E; ++i) v[i] = to_f32(src[i]);
-    if (is_v ? rotate_values : rotate_keys) wave_rotate<D>(v, signs_right, signs_left, sqrt_d);
-    const float* bnd = is_v ? value_bnd : key_bnd;
+    if (is_v ? a.rotate_values : a.rotate_keys) wave_rotate<D>(v, a.signs_right, a.signs_left, a.sqrt_d);
+    const float* bnd = is_v ? a.value_bnd : a.key_bnd;
     if constexpr (SCALED) {
       float ss = 0.f;
 #pragma unroll
@@ -144,8 +493,8 @@ __global__ __launch_bounds__(kBlock) void append_kernel(
       for (int i = 0; i < E; ++i) v[i] = v[i] / scale;
     }
     if constexpr (DEQUANT) {
-      const float* cent = is_v ? value_cent : key_cent;
-      float* dst = (is_v ? value_out : key_out) + r * D + lane * E;
+      const float* cent = is_v ? a.value_cent : a.key_cent;
+      float* dst = (is_v ? a.value_out : a.key_out) + static_cast<int64_t>(r) * D + lane * E;
 #pragma unroll
       for (int i = 0; i < E; ++i) dst[i] = SCALED ? cent[quantize_count<BITS>(v[i], bnd)] * scale
                                                   : cent[quantize_count<BITS>(v[i], bnd)];
@@ -158,10 +507,10 @@ __global__ __launch_bounds__(kBlock) void append_kernel(
     __syncthreads();
     if (active && lane < W) {
       const uint32_t word = pack_word<BITS, D>(s_codes[wave], lane);
-      const int64_t lh = r / seq_new, t = r - lh * seq_new;
-      uint32_t* dst = (is_v ? value_codes : key_codes) + (lh * capacity + offset + t) * W + lane;
-      *dst = word;
-      if (SCALED && lane == 0) (is_v ? value_scales : key_scales)[lh * capacity + offset + t] = scale;
+      const uint32_t lh = a.seq_new.quot(r), t = r - lh * a.seq_new.d;
+      const int64_t slot = static_cast<int64_t>(lh) * a.capacity + a.offset + t;
+      (is_v ? a.value_codes : a.key_codes)[slot * W + lane] = word;
+      if (SCALED && lane == 0) (is_v ? a.value_scales : a.key_scales)[slot] = scale;
     }
   }
 }
@@ -1879,26 +2228,52 @@ template <int D, int BITS, typename T, bool DQ, bool SC>
 int launch_append_part(const AppendParams& p, int64_t g0, int64_t t0, int64_t seq_part, int64_t rows,
                        hipStream_t stream) {
   constexpr int W = D * BITS / 32;
+  constexpr int RPB = kBlock / (D / 16);
   const int64_t row0 = g0 * p.seq_new + t0;
-  const int64_t nblk = (rows * p.streams + kWavesPerBlock - 1) / kWavesPerBlock;
-  hipLaunchKernelGGL((append_kernel<D, BITS, T, DQ, SC>), dim3(static_cast<unsigned>(nblk)), dim3(kBlock), 0, stream,
-                     static_cast<const T*>(p.keys) + row0 * D, static_cast<const T*>(p.values) + row0 * D, rows,
-                     p.streams, seq_part, p.rotate_keys, p.rotate_values, p.signs_left, p.signs_right, sqrt_f32(D),
-                     p.key_bnd, p.value_bnd, p.key_cent, p.value_cent,
-                     p.key_codes ? p.key_codes + g0 * p.capacity * W : nullptr,
-                     p.value_codes ? p.value_codes + g0 * p.capacity * W : nullptr, p.capacity, p.offset + t0,
-                     p.key_out ? p.key_out + row0 * D : nullptr, p.value_out ? p.value_out + row0 * D : nullptr,
-                     p.key_scales ? p.key_scales + g0 * p.capacity : nullptr,
-                     p.value_scales ? p.value_scales + g0 * p.capacity : nullptr);
+  AppendArgs a{};
+  a.keys = static_cast<const T*>(p.keys) + row0 * D;
+  a.values = static_cast<const T*>(p.values) + row0 * D;
+  a.rows = static_cast<uint32_t>(rows);
+  a.seq_new = make_fast_div(static_cast<uint32_t>(seq_part));
+  a.rotate_keys = p.rotate_keys;
+  a.rotate_values = p.rotate_values;
+  a.signs_left = p.signs_left;
+  a.signs_right = p.signs_right;
+  a.sqrt_d = sqrt_f32(D);
+  a.key_bnd = p.key_bnd;
+  a.value_bnd = p.value_bnd;
+  a.key_cent = p.key_cent;
+  a.value_cent = p.value_cent;
+  a.key_codes = p.key_codes ? p.key_codes + g0 * p.capacity * W : nullptr;
+  a.value_codes = p.value_codes ? p.value_codes + g0 * p.capacity * W : nullptr;
+  a.capacity = p.capacity;
+  a.offset = p.offset + t0;
+  a.key_out = p.key_out ? p.key_out + row0 * D : nullptr;
+  a.value_out = p.value_out ? p.value_out + row0 * D : nullptr;
+  a.key_scales = p.key_scales ? p.key_scales + g0 * p.capacity : nullptr;
+  a.value_scales = p.value_scales ? p.value_scales + g0 * p.capacity : nullptr;
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(a.keys) | reinterpret_cast<uintptr_t>(a.values) |
+                         reinterpret_cast<uintptr_t>(a.key_out) | reinterpret_cast<uintptr_t>(a.value_out);
+  a.wide = bits % 16 == 0;
+  if (rows * p.streams <= kAppendFewRows) {
+    const unsigned few = static_cast<unsigned>((rows + kWavesPerBlock - 1) / kWavesPerBlock);
+    hipLaunchKernelGGL((append_few_kernel<D, BITS, T, DQ, SC>), dim3(few, p.streams), dim3(kBlock), 0, stream, a);
+    return launch_status("append_few_kernel");
+  }
+  const int64_t nblk = std::min<int64_t>((rows + RPB - 1) / RPB, kAppendMaxBlocks / p.streams);
+  hipLaunchKernelGGL((append_kernel<D, BITS, T, DQ, SC>), dim3(static_cast<unsigned>(nblk), p.streams), dim3(kBlock),
+                     0, stream, a);
   return launch_status("append_kernel");
 }
 
-// rows = groups * seq_new items per stream; at most kMaxLaunchBlocks
-// workgroups per launch, cut at whole groups, or at tokens when one group
-// alone is larger.
+// rows = groups * seq_new items per stream; at most kMaxAppendRows rows per
+// launch (row numbers are 32-bit), cut at whole groups, or at tokens when one
+// group alone is larger.
+constexpr int64_t kMaxAppendRows = int64_t(1) << 30;
+
 template <int D, int BITS, typename T, bool DQ, bool SC>
 int launch_append(const AppendParams& p, hipStream_t stream) {
-  const int64_t max_rows = kMaxLaunchBlocks * kWavesPerBlock / p.streams;
+  const int64_t max_rows = kMaxAppendRows;
   const int64_t groups = p.rows / p.seq_new;
   if (p.seq_new <= max_rows) {
     const int64_t per = max_rows / p.seq_new;
