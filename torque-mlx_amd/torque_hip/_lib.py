@@ -148,8 +148,7 @@ _NOT_STATUS = {"tq_abi_version", "tq_last_error", "tq_decode_workspace_bytes", "
 
 def call(name: str, *args) -> int:
     """Call an entry point; negative int results raise (ValueError / TorqueHIPError)."""
-    fn = getattr(load(), name)
-    rc = fn(*args)
+    rc = getattr(_LIB or load(), name)(*args)
     if name not in _NOT_STATUS and rc < 0:
         check(rc)
     return rc

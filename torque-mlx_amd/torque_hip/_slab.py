@@ -52,8 +52,8 @@ class SlabStore:
         self.growth_factor = growth_factor
         self.capacity = initial_capacity
         shape = (config.num_layers, config.kv_heads, initial_capacity, self.layout.packed_words)
-        self.key_codes = torch.zeros(shape, dtype=torch.int32, device=dev)
-        self.value_codes = torch.zeros_like(self.key_codes)
+        self._codes = torch.zeros((2, *shape), dtype=torch.int32, device=dev)  # one fill clears both streams
+        self.key_codes, self.value_codes = self._codes[0], self._codes[1]
         self.scaled = config.scale_mode == "rms"
         self.key_scales = torch.zeros(shape[:3], dtype=torch.float32, device=dev) if self.scaled else None
         self.value_scales = torch.zeros(shape[:3], dtype=torch.float32, device=dev) if self.scaled else None
@@ -73,11 +73,10 @@ class SlabStore:
         while new_capacity < min_capacity:
             new_capacity *= self.growth_factor
         shape = (self.config.num_layers, self.config.kv_heads, new_capacity, self.layout.packed_words)
-        new_k = torch.zeros(shape, dtype=torch.int32, device=self.device)
-        new_v = torch.zeros_like(new_k)
-        new_k[:, :, : self.length].copy_(self.key_codes[:, :, : self.length])
-        new_v[:, :, : self.length].copy_(self.value_codes[:, :, : self.length])
-        self.key_codes, self.value_codes = new_k, new_v
+        new = torch.zeros((2, *shape), dtype=torch.int32, device=self.device)
+        new[:, :, :, : self.length].copy_(self._codes[:, :, :, : self.length])
+        self._codes = new
+        self.key_codes, self.value_codes = new[0], new[1]
         if self.scaled:
             new_ks = torch.zeros(shape[:3], dtype=torch.float32, device=self.device)
             new_vs = torch.zeros_like(new_ks)
@@ -88,8 +87,7 @@ class SlabStore:
 
     def reset(self) -> None:
         self.length = 0
-        self.key_codes.zero_()
-        self.value_codes.zero_()
+        self._codes.zero_()
         if self.scaled:
             self.key_scales.zero_()
             self.value_scales.zero_()

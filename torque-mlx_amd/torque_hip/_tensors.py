@@ -12,13 +12,17 @@ from torque_hip._lib import TQ_F16, TQ_F32
 
 
 def device() -> torch.device:
-    if not torch.cuda.is_available():
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         raise RuntimeError("torque_hip needs a HIP device (torch.cuda.is_available() is False)")
     return torch.device("cuda", torch.cuda.current_device())
 
 
 def stream_handle(dev: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The current stream's handle, without the ``torch.cuda.Stream`` object that ``current_stream`` builds."""
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(dev).cuda_stream
+    index = dev.index if dev is not None and dev.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -33,6 +37,13 @@ def to_device(values: Any, dev: torch.device, *, keep_f16: bool = True) -> torch
     """Contiguous, 16-byte aligned device tensor, float32 (float16 kept when allowed)."""
     if isinstance(values, torch.Tensor):
         t = values
+        if (
+            (t.dtype is torch.float32 or (keep_f16 and t.dtype is torch.float16))
+            and t.device == dev
+            and t.is_contiguous()
+            and t.data_ptr() % 16 == 0
+        ):
+            return t
         if t.dtype not in (torch.float32, torch.float16) or (t.dtype == torch.float16 and not keep_f16):
             t = t.to(torch.float32)
         t = t.to(dev).contiguous()
@@ -48,9 +59,9 @@ def to_device(values: Any, dev: torch.device, *, keep_f16: bool = True) -> torch
 
 
 def dtype_code(t: torch.Tensor) -> int:
-    if t.dtype == torch.float16:
+    if t.dtype is torch.float16:
         return TQ_F16
-    if t.dtype == torch.float32:
+    if t.dtype is torch.float32:
         return TQ_F32
     raise ValueError(f"unsupported dtype {t.dtype}")
 
@@ -77,5 +88,5 @@ def codes_to_numpy(t: torch.Tensor) -> np.ndarray:
 
 def shape_of(values: Any) -> tuple[int, ...]:
     if isinstance(values, torch.Tensor):
-        return tuple(int(s) for s in values.shape)
+        return tuple(values.shape)
     return tuple(np.shape(values))

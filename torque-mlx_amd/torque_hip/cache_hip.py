@@ -285,13 +285,19 @@ class TorqueKVCacheHIP:
         profile = self.last_decode_profile if self.profile_decode_components else None
         if self._staged_profile(profile):
             return self._decode_staged(queries, profile)
-        with EventTimer(profile, "packed_decode_seconds", self._store.device):
+
+        def decode() -> torch.Tensor:
             return self._store.decode(
                 queries,
                 rotate_query=self.rotate_queries_on_decode,
                 inverse_output=not self.config.fused_weights,
                 n_splits=self._n_splits(),
             )
+
+        if profile is None:
+            return decode()
+        with EventTimer(profile, "packed_decode_seconds", self._store.device):
+            return decode()
 
     def _decode_staged(self, queries: torch.Tensor, profile: dict[str, float]) -> torch.Tensor:
         """The reference's three-stage split path (cache_mlx.py:752-775), each stage timed."""

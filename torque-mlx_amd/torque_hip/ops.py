@@ -8,6 +8,7 @@ torch tensors on the current HIP device.  Shapes, argument names and the
 
 from __future__ import annotations
 
+from functools import lru_cache
 from math import sqrt
 from typing import Any
 
@@ -51,11 +52,11 @@ class Workspace:
     calls ordered on one stream can share it.
     """
 
-    _pool: dict[tuple[str, int], torch.Tensor] = {}
+    _pool: dict[tuple[torch.device, int], torch.Tensor] = {}
 
     @classmethod
     def get(cls, nbytes: int, dev: torch.device) -> torch.Tensor:
-        key = (str(dev), stream_handle(dev))
+        key = (dev, stream_handle(dev))
         buf = cls._pool.get(key)
         if buf is None or buf.numel() < nbytes:
             if buf is not None:
@@ -65,6 +66,7 @@ class Workspace:
         return buf
 
 
+@lru_cache(maxsize=None)
 def num_cus(dev: torch.device) -> int:
     return int(torch.cuda.get_device_properties(dev).multi_processor_count)
 
@@ -86,9 +88,14 @@ def plan_splits(
     )
 
 
+@lru_cache(maxsize=256)
+def _workspace_bytes(num_layers: int, kv_heads: int, query_heads: int, head_dim: int, n_splits: int, cus: int) -> int:
+    return int(_lib.call("tq_decode_workspace_bytes", num_layers, kv_heads, query_heads, head_dim, n_splits, cus))
+
+
 def workspace_for(num_layers: int, kv_heads: int, query_heads: int, head_dim: int, n_splits: int, dev: torch.device) -> torch.Tensor:
-    nbytes = _lib.call("tq_decode_workspace_bytes", num_layers, kv_heads, query_heads, head_dim, n_splits, num_cus(dev))
-    return Workspace.get(int(nbytes), dev)
+    """A workspace of ``n_splits`` splits (0: of the default plan at any length)."""
+    return Workspace.get(_workspace_bytes(num_layers, kv_heads, query_heads, head_dim, n_splits, num_cus(dev)), dev)
 
 
 def packed_decode(
@@ -133,9 +140,7 @@ def packed_decode(
     flags = (_lib.TQ_ROTATE_QUERY if rotate_query else 0) | (_lib.TQ_INVERSE_OUTPUT if inverse_output else 0)
     flags |= _lib.TQ_F32_PRODUCTS if f32_products or scaled else 0
     flags |= _lib.TQ_MATRIX_PRODUCTS if matrix_products else 0
-    if n_splits is None or n_splits <= 0:
-        n_splits = plan_splits(num_layers, kv_heads, query_heads, head_dim, seq_len, dev, bit_width=bit_width,
-                               flags=flags)
+    n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
     ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
     if out is None:
         out = torch.empty((num_layers, query_heads, head_dim), dtype=torch.float32, device=dev)
@@ -209,9 +214,7 @@ def packed_decode_append(
     append_flags = (_lib.TQ_ROTATE_KEYS if rotate_keys else 0) | (_lib.TQ_ROTATE_VALUES if rotate_values else 0)
     decode_flags = (_lib.TQ_ROTATE_QUERY if rotate_query else 0) | (_lib.TQ_INVERSE_OUTPUT if inverse_output else 0)
     decode_flags |= _lib.TQ_MATRIX_PRODUCTS if matrix_products else 0
-    if n_splits is None or n_splits <= 0:
-        n_splits = plan_splits(num_layers, kv_heads, query_heads, head_dim, seq_len, dev, bit_width=bit_width,
-                               flags=decode_flags)
+    n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
     ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
     if out is None:
         out = torch.empty((num_layers, query_heads, head_dim), dtype=torch.float32, device=dev)
@@ -268,8 +271,7 @@ def dense_decode(
 ) -> torch.Tensor:
     """One ``tq_decode_dense`` launch: dense fp16/fp32 K/V slabs [L, Hkv, capacity, D]."""
     dev = query.device
-    if n_splits is None or n_splits <= 0:
-        n_splits = plan_splits(num_layers, kv_heads, query_heads, head_dim, seq_len, dev)
+    n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
     ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
     if out is None:
         out = torch.empty((num_layers, query_heads, head_dim), dtype=torch.float32, device=dev)
