@@ -1,0 +1,42 @@
+"""The default split plan of calls with many units, on the host: sizes that callers rely on."""
+
+from __future__ import annotations
+
+import random
+
+import pytest
+
+from torque_hip import _lib
+
+CUS = 256
+SCRATCH = 8 << 20  # tq_decode_noalloc's
+
+
+def _splits(layers, kv, group, dim, bits, flags, seq):
+    return _lib.call("tq_decode_default_splits", layers, kv, kv * group, dim, bits, flags, seq, CUS)
+
+
+def _bytes(layers, kv, group, dim, n):
+    return _lib.call("tq_decode_workspace_bytes", layers, kv, kv * group, dim, n, CUS)
+
+
+def test_default_workspace_covers_every_plan():
+    rng = random.Random(0)
+    for _ in range(5000):
+        shape = (rng.choice([1, 2, 3, 6, 12, 16, 24, 32, 64]), rng.choice([1, 2, 4, 8]), rng.randint(1, 8), rng.choice([64, 128, 256]))
+        n = _splits(*shape, rng.choice([0, 2, 3, 4]), rng.choice([0, _lib.TQ_F32_PRODUCTS]), int(10 ** rng.uniform(0, 5.3)))
+        need = _bytes(*shape, n)
+        assert need <= _bytes(*shape, 0)
+        if n > 1:  # more than the scratch holds only where one split does not fit either
+            assert need <= SCRATCH or _bytes(*shape, 1) > SCRATCH, (shape, n)
+
+
+@pytest.mark.parametrize("layers,kv,group,dim,bits,seq,most", [
+    (24, 8, 4, 128, 3, 8192, 4),  # 192 units: 3 workgroups to a CU
+    (24, 8, 1, 128, 4, 8192, 4),
+    (24, 4, 4, 256, 3, 8192, 5),  # one round, 480 workgroups: more splits would save less than 1/16
+    (1, 8, 4, 128, 3, 32768, 64),  # one round fills the CUs evenly: unchanged
+    (24, 8, 1, 128, 4, 200, 2),  # too short for more
+])
+def test_workgroups_spread_over_the_cus(layers, kv, group, dim, bits, seq, most):
+    assert _splits(layers, kv, group, dim, bits, 0, seq) == most

@@ -1598,6 +1598,37 @@ struct Plan {
 
 constexpr int kMinTokensPerSplit = 128;
 
+// Most workgroups per CU of a plan whose workgroups do not all run at once
+// (see balanced_splits), and the work of a workgroup besides its blocks, in
+// blocks.
+constexpr int kMaxLoad = 6;
+constexpr int kLoadOverhead = 5;
+constexpr int kMergeWork = 12;  // the merge launch that more than one split adds
+
+// Splits of a call with many units.  One resident round of workgroups leaves
+// CUs with one workgroup less than others when units does not divide it (192
+// units: 384 workgroups, 2 on half of the CUs and 1 on the rest); a CU works
+// through its workgroups at the same rate whether one or two are resident, so
+// what counts is the work of the CU with the most.  Starting from the
+// one-round count ns0, take the count that makes it smallest, if that is at
+// least 1/16 less.  Measured on MI355X, 24 layers x 8 KV heads: 3-bit rows at
+// head_dim 128 x 8192 tokens, groups of 4, 75 us at 2 splits, 59 at 4 (768
+// workgroups, 3 to a CU), 64 at 5, 63 at 8; 4-bit rows, groups of 1, 60, 47,
+// 50, 47; at head_dim 64, groups of 2, 38, 31, 33, 31.  Over 20 random shapes
+// whose count it changes: 1.08 to 1.66 times as fast.  The overheads keep it
+// from short sequences, where more splits lose (640 units x 2235 tokens at
+// head_dim 256: 65 us at 1 split, 67.5 at 2).
+int balanced_splits(int units, int ns0, int64_t blocks, int num_cus) {
+  auto work = [&](int64_t ns) {
+    return ((units * ns + num_cus - 1) / num_cus) * (kLoadOverhead + (blocks + ns - 1) / ns) + (ns > 1 ? kMergeWork : 0);
+  };
+  int best = ns0;
+  const int64_t most = std::min<int64_t>({static_cast<int64_t>(kMaxLoad) * num_cus / units, blocks, kMaxSplits});
+  for (int64_t ns = ns0 + 1; ns <= most; ++ns)
+    if (16 * work(ns) <= 15 * work(ns0) && work(ns) < work(best)) best = static_cast<int>(ns);
+  return best;
+}
+
 int default_splits(int units, int64_t seq_len, int num_cus, int wgs_per_cu) {
   if (num_cus <= 0) num_cus = 256;
   const int64_t target = static_cast<int64_t>(wgs_per_cu) * num_cus;
@@ -1764,7 +1795,16 @@ KernelChoice choose_kernel(int units, int64_t seq_len, int n_splits, int fmt, in
     if ((flags & TQ_MATRIX_PRODUCTS) != 0 || blocks / std::min<int64_t>(blocks, ns) >= mx_min_blocks_per_split(head_dim))
       return {SplitKernel::Mx, ns};
   }
-  return {SplitKernel::Fp32, n_splits > 0 ? n_splits : default_splits(units, seq_len, num_cus, 2)};
+  if (n_splits > 0) return {SplitKernel::Fp32, n_splits};
+  if (num_cus <= 0) num_cus = 256;
+  const int ns0 = default_splits(units, seq_len, num_cus, 2);
+  // one split per kMinTokensPerSplit tokens at most, as in default_splits
+  const int64_t by_len = (seq_len + kMinTokensPerSplit - 1) / kMinTokensPerSplit;
+  if (ns0 >= by_len) return {SplitKernel::Fp32, ns0};
+  const bool packed = fmt == 2 || fmt == 3 || fmt == 4;
+  const int64_t rows = decode_block_rows(packed ? fmt : 16, head_dim);  // dense rows: one plan for both types
+  const int ns = balanced_splits(units, ns0, (seq_len + rows - 1) / rows, num_cus);
+  return {SplitKernel::Fp32, static_cast<int>(std::min<int64_t>(ns, by_len))};
 }
 
 // Fills the split plan of a decode call over `fmt` rows (see
@@ -2647,8 +2687,12 @@ size_t tq_decode_workspace_bytes(int num_layers, int kv_heads, int query_heads, 
   const int hg = pick_hg(group);
   const int units = num_layers * kv_heads * (group / hg);
   int ns = n_splits;
-  // the larger of the two split kernels' defaults (two workgroups per CU)
-  if (ns <= 0) ns = default_splits(units, static_cast<int64_t>(kMaxSplits) * kMinTokensPerSplit, num_cus, 2);
+  // the larger of the two split kernels' defaults (two workgroups per CU, or
+  // kMaxLoad where they are not all resident at once)
+  if (ns <= 0) {
+    ns = default_splits(units, static_cast<int64_t>(kMaxSplits) * kMinTokensPerSplit, num_cus, 2);
+    ns = std::max(ns, kMaxLoad * (num_cus > 0 ? num_cus : 256) / units);
+  }
   ns = std::min(ns, kMaxSplits);
   return workspace_layout(static_cast<int64_t>(num_layers) * query_heads, static_cast<int64_t>(num_layers) * kv_heads,
                           head_dim, ns)
