@@ -42,7 +42,7 @@ enum {
   TQ_ERR_LAUNCH = -3       /* HIP launch failure (Python: RuntimeError) */
 };
 
-enum { TQ_F32 = 0, TQ_F16 = 1 };
+enum { TQ_F32 = 0, TQ_F16 = 1, TQ_BF16 = 2 /* tq_rotary and tq_unrotate_gate only */ };
 
 /* tq_append / tq_quantize_dequantize flags (reference cache_mlx.py:52-54) */
 enum { TQ_ROTATE_KEYS = 1, TQ_ROTATE_VALUES = 2 };
@@ -303,6 +303,28 @@ int tq_softmax_rows(const float* scores, int batch, int64_t seq_len, float scale
  * Replaces accumulate_packed_values_batched (mlx_ops.py:148-178, 534-568). */
 int tq_accumulate_packed(const float* weights, const uint32_t* codes, int batch, int64_t seq_len, int head_dim,
                          int bits, const float* centroids, float* out, hipStream_t stream);
+
+/* Rotary embedding of one layer's queries and keys (reference qwen_mlx.py:800-812,
+ * the model's rope in rotate-half form): out = x cos + rotate_half(x) sin on
+ * the first rotary_dim (even) of head_dim dimensions, the others copied, each
+ * operation rounded to out_dtype.  query / key rows [heads, tokens, head_dim]
+ * in x_dtype with the given element strides and unit stride along head_dim;
+ * cos / sin [tokens, rotary_dim] in table_dtype, rows *_stride apart;
+ * query_out / key_out contiguous [heads, tokens, head_dim]. */
+int tq_rotary(const void* query, const void* key, int x_dtype, int query_heads, int key_heads, int64_t tokens,
+              int head_dim, int64_t q_head_stride, int64_t q_token_stride, int64_t k_head_stride,
+              int64_t k_token_stride, const void* cos, const void* sin, int table_dtype, int64_t cos_stride,
+              int64_t sin_stride, int rotary_dim, void* query_out, void* key_out, int out_dtype, hipStream_t stream);
+
+/* Attention output to output-projection input (reference qwen_mlx.py:621-630,
+ * 855-864): inverse rotation of every float32 head row of attn [heads,
+ * tokens, head_dim] (element strides, unit stride along head_dim), times
+ * sigmoid(gate) in float32, rounded to out_dtype into contiguous out [tokens,
+ * heads * head_dim].  gate: the same rows in gate_dtype with its own strides. */
+int tq_unrotate_gate(const float* attn, int heads, int64_t tokens, int head_dim, int64_t head_stride,
+                     int64_t token_stride, const void* gate, int gate_dtype, int64_t gate_head_stride,
+                     int64_t gate_token_stride, const float* signs_left, const float* signs_right, void* out,
+                     int out_dtype, hipStream_t stream);
 
 /* Measurement helper, no counterpart in the reference: streams `bytes` bytes
  * (a multiple of 16, 16-byte aligned) through nontemporal 16-byte loads,

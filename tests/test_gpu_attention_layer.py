@@ -1,0 +1,84 @@
+"""The adapter's rotary and gate kernels against the torch operations they stand for."""
+
+from __future__ import annotations
+
+import itertools
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [torch.float32, torch.float16, torch.bfloat16]
+
+
+def _rotary_reference(x, cos, sin):
+    r = cos.shape[-1]
+    a, rest = x[..., :r], x[..., r:]
+    half = torch.cat((-a[..., r // 2:], a[..., : r // 2]), dim=-1)
+    return torch.cat([a * cos[:, None] + half * sin[:, None], rest], dim=-1)
+
+
+@pytest.mark.parametrize("head_dim,rotary_dim", [(64, 64), (64, 2), (128, 32), (256, 64), (256, 130)])
+@pytest.mark.parametrize("tokens,q_heads,k_heads", [(1, 4, 1), (37, 5, 2)])
+def test_rotary_bit_exact(hip_device, head_dim, rotary_dim, tokens, q_heads, k_heads):
+    from torque_hip import qwen_torch as qt
+
+    g = torch.Generator(device=hip_device).manual_seed(head_dim + rotary_dim + tokens)
+    for x_type, table_type in itertools.product(TYPES, TYPES):
+        q, k = (torch.randn(1, tokens, h, head_dim + 3, generator=g, device=hip_device).to(x_type)[..., 1 : 1 + head_dim].transpose(1, 2)
+                for h in (q_heads, k_heads))
+        cos, sin = (torch.randn(1, tokens, rotary_dim, generator=g, device=hip_device).to(table_type) for _ in range(2))
+        got = qt._rotary_fused(q, k, cos, sin)
+        assert got is not None
+        for y, x in zip(got, (q, k)):
+            expected = _rotary_reference(x, cos, sin)
+            assert y.dtype == expected.dtype and y.is_contiguous()
+            assert torch.equal(y, expected), (x_type, table_type)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize("tokens,heads", [(1, 4), (37, 5)])
+def test_unrotate_gate(hip_device, head_dim, tokens, heads):
+    """Two float32 operations after the bit-identical rotation, and a sigmoid of two more: the result is within 4 ulp
+    (4 x 2^-23) of the torch composition in float32, one unit of the output type more where that rounds."""
+    from torque_hip import RotationSpec
+    from torque_hip import qwen_torch as qt
+
+    rotation = RotationSpec.from_seed(head_dim, 3)
+    g = torch.Generator(device=hip_device).manual_seed(head_dim + tokens)
+    for gate_type, out_type in itertools.product(TYPES, TYPES):
+        attn = torch.randn(1, tokens, heads, head_dim, generator=g, device=hip_device).transpose(1, 2)
+        both = 4.0 * torch.randn(1, tokens, heads, 2 * head_dim, generator=g, device=hip_device)
+        gate = both.to(gate_type)[..., head_dim:]
+        got = qt._unrotate_gate(attn, gate, rotation=rotation, dtype=out_type)
+        rotated = qt.runtime_unrotate_attention_output(attn, rotation=rotation)
+        expected = rotated.transpose(1, 2).reshape(1, tokens, -1) * torch.sigmoid(gate.reshape(1, tokens, -1).float())
+        assert got.dtype == out_type and got.shape == expected.shape
+        unit = {torch.float32: 0.0, torch.float16: 2.0**-10, torch.bfloat16: 2.0**-7}[out_type]
+        torch.testing.assert_close(got.float(), expected, rtol=4 * 2.0**-23 + unit, atol=1e-7 if unit else 1e-30)
+
+
+def test_gradients_and_transforms_keep_the_torch_operations(hip_device):
+    from torque_hip import RotationSpec
+    from torque_hip import qwen_torch as qt
+
+    q, k = torch.randn(1, 2, 3, 64, device=hip_device), torch.randn(1, 1, 3, 64, device=hip_device)
+    cos, sin = torch.randn(1, 3, 16, device=hip_device), torch.randn(1, 3, 16, device=hip_device)
+    want = _rotary_reference(q, cos, sin)
+    leaf = q.clone().requires_grad_()
+    out = qt.apply_rotary(leaf, k, cos, sin)[0]
+    assert out.requires_grad and torch.equal(out, want)
+    with torch.no_grad():
+        assert qt._rotary_fused(leaf, k, cos, sin) is not None
+    stacked = torch.func.vmap(lambda x: qt.apply_rotary(x, k, cos, sin)[0])(torch.stack([q, q]))
+    assert torch.equal(stacked[1], want)
+    tangent = torch.func.jvp(lambda x: qt.apply_rotary(x, k, cos, sin)[0], (q,), (torch.ones_like(q),))[1]
+    assert torch.allclose(tangent, _rotary_reference(torch.ones_like(q), cos, sin))
+    assert qt._rotary_fused(q.cpu(), k.cpu(), cos.cpu(), sin.cpu()) is None
+    assert qt._rotary_fused(q.double(), k.double(), cos, sin) is None
+    assert all(torch.equal(a, b) for a, b in zip(qt.apply_rotary(q, k, cos[..., :0], sin[..., :0]), (q, k)))
+    gate = torch.randn(1, 3, 2, 64, device=hip_device, requires_grad=True)
+    rotation = RotationSpec.from_seed(64, 1)
+    qt._unrotate_gate(q, gate, rotation=rotation, dtype=torch.float32).sum().backward()
+    assert gate.grad is not None and gate.grad.abs().sum() > 0

@@ -1540,6 +1540,11 @@ __global__ __launch_bounds__(kBlock) void accumulate_kernel(const float* __restr
   }
 }
 
+// ============================================================== attention layer
+
+
+#include "attention_layer.hpp"
+
 // ============================================================== measurement
 
 
@@ -2864,6 +2869,73 @@ int tq_accumulate_packed(const float* weights, const uint32_t* codes, int batch,
   if (!weights || !codes || !centroids || !out) return fail(TQ_ERR_BAD_ARG, "null pointer argument");
   return with_d<StageBody>(head_dim, 2, bits, weights, reinterpret_cast<const uint8_t*>(codes), batch, seq_len,
                            centroids, out, stream);
+}
+
+int tq_rotary(const void* query, const void* key, int x_dtype, int query_heads, int key_heads, int64_t tokens,
+              int head_dim, int64_t q_head_stride, int64_t q_token_stride, int64_t k_head_stride,
+              int64_t k_token_stride, const void* cos, const void* sin, int table_dtype, int64_t cos_stride,
+              int64_t sin_stride, int rotary_dim, void* query_out, void* key_out, int out_dtype, hipStream_t stream) {
+  if (query_heads < 0 || key_heads < 0 || tokens < 0 || head_dim <= 0)
+    return fail(TQ_ERR_BAD_ARG, "heads and tokens must be non-negative, head_dim positive");
+  if (rotary_dim < 0 || rotary_dim % 2 != 0 || rotary_dim > head_dim)
+    return fail(TQ_ERR_BAD_ARG, "rotary_dim must be even and at most head_dim");
+  for (int type : {x_dtype, table_dtype, out_dtype})
+    if (type < TQ_F32 || type > TQ_BF16) return fail(TQ_ERR_BAD_ARG, "dtypes must be F32, F16 or BF16");
+  const int64_t rows = (static_cast<int64_t>(query_heads) + key_heads) * tokens;
+  if (rows == 0) return TQ_OK;
+  if (!query || !key || !cos || !sin || !query_out || !key_out) return fail(TQ_ERR_BAD_ARG, "null pointer argument");
+  if (tokens > INT32_MAX || (rows + kWavesPerBlock - 1) / kWavesPerBlock > ((int64_t(1) << 32) - 1) / kBlock)
+    return fail(TQ_ERR_BAD_ARG, "heads x tokens exceeds one launch");
+  RotaryArgs a{};
+  a.x[0] = {query, x_dtype, query_heads, q_head_stride, q_token_stride};
+  a.x[1] = {key, x_dtype, key_heads, k_head_stride, k_token_stride};
+  a.out[0] = query_out;
+  a.out[1] = key_out;
+  a.out_type = out_dtype;
+  a.cos = cos;
+  a.sin = sin;
+  a.table_type = table_dtype;
+  a.cos_stride = cos_stride;
+  a.sin_stride = sin_stride;
+  a.tokens = static_cast<int>(tokens);
+  a.head_dim = head_dim;
+  a.rotary_dim = rotary_dim;
+  const unsigned nblk = static_cast<unsigned>((rows + kWavesPerBlock - 1) / kWavesPerBlock);
+  hipLaunchKernelGGL(rotary_kernel, dim3(nblk), dim3(kBlock), 0, stream, a);
+  return launch_status("rotary_kernel");
+}
+
+int tq_unrotate_gate(const float* attn, int heads, int64_t tokens, int head_dim, int64_t head_stride,
+                     int64_t token_stride, const void* gate, int gate_dtype, int64_t gate_head_stride,
+                     int64_t gate_token_stride, const float* signs_left, const float* signs_right, void* out,
+                     int out_dtype, hipStream_t stream) {
+  const int rc = check_geometry(head_dim, 0);
+  if (rc) return rc;
+  if (heads < 0 || tokens < 0) return fail(TQ_ERR_BAD_ARG, "heads and tokens must be non-negative");
+  for (int type : {gate_dtype, out_dtype})
+    if (type < TQ_F32 || type > TQ_BF16) return fail(TQ_ERR_BAD_ARG, "dtypes must be F32, F16 or BF16");
+  const int64_t rows = heads * tokens;
+  if (rows == 0) return TQ_OK;
+  if (!attn || !gate || !signs_left || !signs_right || !out) return fail(TQ_ERR_BAD_ARG, "null pointer argument");
+  if (tokens > INT32_MAX || (rows + kWavesPerBlock - 1) / kWavesPerBlock > ((int64_t(1) << 32) - 1) / kBlock)
+    return fail(TQ_ERR_BAD_ARG, "heads x tokens exceeds one launch");
+  GateArgs a{};
+  a.attn = {attn, kTypeF32, heads, head_stride, token_stride};
+  a.gate = {gate, gate_dtype, heads, gate_head_stride, gate_token_stride};
+  a.out = out;
+  a.out_type = out_dtype;
+  a.tokens = static_cast<int>(tokens);
+  a.signs_left = signs_left;
+  a.signs_right = signs_right;
+  a.sqrt_d = sqrt_f32(head_dim);
+  const dim3 grid(static_cast<unsigned>((rows + kWavesPerBlock - 1) / kWavesPerBlock));
+  if (head_dim == 64)
+    hipLaunchKernelGGL(unrotate_gate_kernel<64>, grid, dim3(kBlock), 0, stream, a);
+  else if (head_dim == 128)
+    hipLaunchKernelGGL(unrotate_gate_kernel<128>, grid, dim3(kBlock), 0, stream, a);
+  else
+    hipLaunchKernelGGL(unrotate_gate_kernel<256>, grid, dim3(kBlock), 0, stream, a);
+  return launch_status("unrotate_gate_kernel");
 }
 
 int tq_stream_read(const void* data, size_t bytes, float* sink, int n_blocks, hipStream_t stream, hipEvent_t start,

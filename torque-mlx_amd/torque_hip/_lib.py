@@ -28,6 +28,7 @@ TQ_ERR_LAUNCH = -3
 
 TQ_F32 = 0
 TQ_F16 = 1
+TQ_BF16 = 2  # tq_rotary and tq_unrotate_gate only
 
 TQ_ROTATE_KEYS = 1
 TQ_ROTATE_VALUES = 2
@@ -96,6 +97,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "tq_score_packed": (_i, [_p, _p, _i, _i64, _i, _i, _p, _p, _p]),
     "tq_softmax_rows": (_i, [_p, _i, _i64, _f, _p, _p]),
     "tq_accumulate_packed": (_i, [_p, _p, _i, _i64, _i, _i, _p, _p, _p]),
+    "tq_rotary": (
+        _i,
+        [_p, _p, _i, _i, _i, _i64, _i, _i64, _i64, _i64, _i64, _p, _p, _i, _i64, _i64, _i, _p, _p, _i, _p],
+    ),
+    "tq_unrotate_gate": (_i, [_p, _i, _i64, _i, _i64, _i64, _p, _i, _i64, _i64, _p, _p, _p, _i, _p]),
     "tq_stream_read": (_i, [_p, _sz, _p, _i, _p, _p, _p]),
 }
 

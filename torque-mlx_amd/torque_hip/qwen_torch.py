@@ -33,7 +33,10 @@ from typing import Any, Callable
 import numpy as np
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
+from torque_hip import _lib
+from torque_hip._tensors import stream_handle
 from torque_hip.cache_hip import TorqueKVCacheHIP
 from torque_hip.config import TorqueConfig
 from torque_hip.quantization import Codebook
@@ -223,9 +226,60 @@ def _rotate_half(x: torch.Tensor) -> torch.Tensor:
     return torch.cat((-x[..., half:], x[..., :half]), dim=-1)
 
 
+_TYPES = {torch.float32: _lib.TQ_F32, torch.float16: _lib.TQ_F16, torch.bfloat16: _lib.TQ_BF16}
+
+
+def _plain(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may read these tensors directly: ordinary tensors of one GPU and a type it takes, with no
+    gradient, transform, trace or dispatch mode to see the operations it stands for."""
+    dev = tensors[0].device
+    for t in tensors:
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return False
+        if t.device != dev or t.dtype not in _TYPES or t.is_neg() or (t.requires_grad and torch.is_grad_enabled()):
+            return False
+    return (
+        dev.type == "cuda"
+        and not torch.compiler.is_compiling()
+        and not torch.jit.is_tracing()
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and forward_ad._current_level < 0
+        and torch._C._len_torch_dispatch_stack() == 0
+        and torch._C._len_torch_function_stack() == 0
+    )
+
+
+def _rotary_fused(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor] | None:
+    """``apply_rotary`` in one launch, or None where the operands are not of the forms ``tq_rotary`` takes."""
+    if not (q.dim() == k.dim() == 4 and cos.dim() == sin.dim() == 3 and cos.shape == sin.shape):
+        return None
+    _, heads, tokens, dim = q.shape
+    r = cos.shape[-1]
+    if (
+        q.shape[0] != 1 or cos.shape[0] != 1 or cos.shape[1] != tokens or k.shape != (1, k.shape[1], tokens, dim)
+        or r % 2 or r > dim or q.dtype != k.dtype or cos.dtype != sin.dtype
+        or 0 in (tokens, r, heads, k.shape[1])  # nothing to rotate
+        or not q.stride(3) == k.stride(3) == cos.stride(2) == sin.stride(2) == 1
+        or not _plain(q, k, cos, sin)
+    ):
+        return None
+    dtype = torch.promote_types(q.dtype, cos.dtype)
+    q_out = torch.empty(q.shape, dtype=dtype, device=q.device)
+    k_out = torch.empty(k.shape, dtype=dtype, device=q.device)
+    _lib.call(
+        "tq_rotary", q.data_ptr(), k.data_ptr(), _TYPES[q.dtype], heads, k.shape[1], tokens, dim, q.stride(1), q.stride(2),
+        k.stride(1), k.stride(2), cos.data_ptr(), sin.data_ptr(), _TYPES[cos.dtype], cos.stride(1), sin.stride(1), r,
+        q_out.data_ptr(), k_out.data_ptr(), _TYPES[dtype], stream_handle(q.device),
+    )
+    return q_out, k_out
+
+
 def apply_rotary(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Rotary embedding on the first ``cos.shape[-1]`` dims of [B, H, L, D] queries and keys (rotate-half
     convention, the rest passed through), ``cos`` / ``sin`` of shape [B, L, rotary_dim]."""
+    fused = _rotary_fused(q, k, cos, sin)
+    if fused is not None:
+        return fused
     cos, sin = cos.unsqueeze(1), sin.unsqueeze(1)
     r = int(cos.shape[-1])
     q_rot, q_pass = q[..., :r], q[..., r:]
@@ -233,6 +287,27 @@ def apply_rotary(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch
     q_out = torch.cat([q_rot * cos + _rotate_half(q_rot) * sin, q_pass], dim=-1)
     k_out = torch.cat([k_rot * cos + _rotate_half(k_rot) * sin, k_pass], dim=-1)
     return q_out, k_out
+
+
+def _unrotate_gate(attn_output: torch.Tensor, gate: torch.Tensor, *, rotation: RotationSpec, dtype: torch.dtype) -> torch.Tensor:
+    """[1, H, L, D] attention output and [1, L, H, D] gate -> the output projection's input [1, L, H * D]:
+    ``runtime_unrotate_attention_output`` times ``sigmoid(gate)`` in float32, in ``dtype``."""
+    _, heads, tokens, dim = attn_output.shape
+    if (
+        attn_output.dtype is torch.float32 and dtype in _TYPES and tokens
+        and attn_output.stride(3) == gate.stride(3) == 1 and _plain(attn_output, gate)
+    ):
+        left, right = rotation.device_signs(attn_output.device)
+        out = torch.empty((1, tokens, heads * dim), dtype=dtype, device=attn_output.device)
+        _lib.call(
+            "tq_unrotate_gate", attn_output.data_ptr(), heads, tokens, dim, attn_output.stride(1), attn_output.stride(2),
+            gate.data_ptr(), _TYPES[gate.dtype], gate.stride(2), gate.stride(1), left.data_ptr(), right.data_ptr(),
+            out.data_ptr(), _TYPES[dtype], stream_handle(attn_output.device),
+        )
+        return out
+    output = runtime_unrotate_attention_output(attn_output, rotation=rotation)
+    output = output.transpose(1, 2).reshape(1, tokens, -1)
+    return (output * torch.sigmoid(gate.reshape(1, tokens, -1).float())).to(dtype)
 
 
 def _dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float, offset: int) -> torch.Tensor:
@@ -286,7 +361,6 @@ class TorqueQwenAttention(torch.nn.Module):
             raise ValueError("Torque HIP Qwen runtime currently supports batch size 1")
         hd = self.head_dim
         queries, gate = torch.chunk(attn.q_proj(hidden_states).view(B, L, -1, hd * 2), 2, dim=-1)
-        gate = gate.reshape(B, L, -1)
         queries = attn.q_norm(queries).transpose(1, 2)
         keys = attn.k_norm(attn.k_proj(hidden_states).view(B, L, -1, hd)).transpose(1, 2)
         values = attn.v_proj(hidden_states).view(B, L, -1, hd).transpose(1, 2)
@@ -307,9 +381,7 @@ class TorqueQwenAttention(torch.nn.Module):
         else:
             output = _dense_attention(queries, keys, values, scale=self.scaling, offset=0)
 
-        output = runtime_unrotate_attention_output(output, rotation=self.rotation)
-        output = output.transpose(1, 2).reshape(B, L, -1)
-        projected = (output * torch.sigmoid(gate.float())).to(attn.o_proj.weight.dtype)
+        projected = _unrotate_gate(output, gate, rotation=self.rotation, dtype=attn.o_proj.weight.dtype)
         return attn.o_proj(projected), None
 
 
