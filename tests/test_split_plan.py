@@ -36,7 +36,14 @@ def test_default_workspace_covers_every_plan():
     (24, 8, 1, 128, 4, 8192, 4),
     (24, 4, 4, 256, 3, 8192, 5),  # one round, 480 workgroups: more splits would save less than 1/16
     (1, 8, 4, 128, 3, 32768, 64),  # one round fills the CUs evenly: unchanged
-    (24, 8, 1, 128, 4, 200, 2),  # too short for more
+    (24, 8, 1, 128, 4, 200, 1),  # short: one launch
+    (1, 8, 1, 128, 4, 512, 1),
+    (1, 8, 1, 128, 4, 513, 5),
+    (1, 4, 4, 256, 4, 256, 1),
+    (1, 4, 4, 256, 4, 257, 3),
+    (1, 4, 4, 64, 3, 512, 1),
+    (1, 4, 4, 64, 3, 513, 5),
+    (1, 8, 1, 128, 0, 512, 4),  # dense rows: as long as any
 ])
 def test_workgroups_spread_over_the_cus(layers, kv, group, dim, bits, seq, most):
     assert _splits(layers, kv, group, dim, bits, 0, seq) == most

@@ -1786,6 +1786,23 @@ bool mx_shape(int fmt, int head_dim, int hg) {
 // workgroup, writing its 128 KB of tables costs more than its loop saves.
 int mx_min_blocks_per_split(int head_dim) { return head_dim == 256 ? 8 : 4; }
 
+// Short packed sequences take one split by default: the workgroup of a head
+// group reads them in 8 iterations at most and finishes its rows itself, so
+// the call is one launch.  Measured on MI355X (one decode on the GPU, then
+// with its Python call): 256 tokens x 8 heads at head_dim 128 6.0 / 8.5 us
+// against 7.4 / 11.4 in 2 splits, 512 tokens 7.8 / 8.6 against 7.3 / 11.6 (in
+// groups of 4, on the matrix kernel, 7.0 / 8.5 against 7.8 / 11.6), 768
+// tokens 9.9 / 9.9 against 7.5 / 11.5; at head_dim 256 256 tokens 8.9 / 9.0
+// against 9.2 / 11.3, 384 tokens 11.2 / 11.2 against 9.3 / 11.4; at head_dim
+// 64 512 tokens 6.5 / 8.6 against 7.3 / 11.2.
+constexpr int kShortBlocks = 8;
+constexpr int kShortTokens = 512;
+
+bool one_split(int64_t seq_len, int fmt, int head_dim) {
+  const bool packed = fmt == 2 || fmt == 3 || fmt == 4;
+  return packed && seq_len <= std::min(kShortTokens, kShortBlocks * decode_block_rows(fmt, head_dim));
+}
+
 // Split kernel and split count of a decode over `units` work units with
 // decode `flags` (n_splits <= 0: the default count for the chosen kernel).
 struct KernelChoice {
@@ -1794,6 +1811,7 @@ struct KernelChoice {
 };
 KernelChoice choose_kernel(int units, int64_t seq_len, int n_splits, int fmt, int head_dim, int hg, int flags,
                            int num_cus) {
+  if (n_splits <= 0 && one_split(seq_len, fmt, head_dim)) n_splits = 1;
   if (mx_shape(fmt, head_dim, hg) && (flags & TQ_F32_PRODUCTS) == 0) {
     const int ns = n_splits > 0 ? n_splits : default_splits(units, seq_len, num_cus, 1);
     const int64_t blocks = std::max<int64_t>(1, (seq_len + mx::kStride - 1) / mx::kStride);
