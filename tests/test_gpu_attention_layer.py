@@ -82,3 +82,50 @@ def test_gradients_and_transforms_keep_the_torch_operations(hip_device):
     rotation = RotationSpec.from_seed(64, 1)
     qt._unrotate_gate(q, gate, rotation=rotation, dtype=torch.float32).sum().backward()
     assert gate.grad is not None and gate.grad.abs().sum() > 0
+
+
+def _check_attention(q, k, v, scale, offset):
+    """Against float64.  A term of a score carries 2^-22 of its size (the splits and the cross term left out) and its
+    float32 sum as much again, so a score is off by at most 2 A 2^-22, A its sum of magnitudes, and every weight by
+    that, relatively, in the numerator and the sum; splits and sums of the values add a few 2^-22.  An output is then
+    within (4 A + 16) 2^-22 of the same weighted sum of the values' magnitudes."""
+    from torque_hip import qwen_torch as qt
+
+    assert qt._prompt_kernel_takes(q, k, v)
+    got = qt._dense_attention(q, k, v, scale=scale, offset=offset)
+    assert got.dtype == torch.float32 and got.shape == q.shape
+    q, k, v = q[0].double(), k[0].double(), v[0].double()
+    group = q.shape[0] // k.shape[0]
+    allowed = torch.arange(k.shape[1], device=q.device)[None] <= torch.arange(offset, offset + q.shape[1], device=q.device)[:, None]
+    for h in range(q.shape[0]):
+        kt, vh = k[h // group].t().contiguous(), v[h // group].contiguous()
+        weights = torch.softmax((torch.matmul(q[h], kt) * scale).masked_fill(~allowed, float("-inf")), dim=-1)
+        most = torch.matmul(q[h].abs(), kt.abs()).max().item() * scale
+        error = (got[0, h] - torch.matmul(weights, vh)).abs()
+        assert torch.all(error <= (4 * most + 16) * 2.0**-22 * torch.matmul(weights, vh.abs()) + 1e-38)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize("tokens,offset,heads,kv_heads", [
+    (1, 0, 1, 1), (2, 0, 4, 4), (16, 0, 5, 1), (17, 15, 6, 2), (31, 1, 8, 2), (33, 64, 7, 7), (130, 3, 16, 4), (257, 0, 3, 1),
+])
+def test_prompt_attention(hip_device, head_dim, tokens, offset, heads, kv_heads):
+    """The edges of a 16-row, 32-key tile, operands of every type, strided rows."""
+    g = torch.Generator(device=hip_device).manual_seed(head_dim + tokens)
+    keys = tokens + offset
+    for types in ((torch.float32,) * 3, (torch.float32, torch.float32, torch.bfloat16), (torch.float16,) * 3):
+        rows = lambda n, h: torch.randn(1, n, h, head_dim + 8, generator=g, device=hip_device)[..., 3 : 3 + head_dim].transpose(1, 2)
+        q, k, v = (x.to(t) for x, t in zip((rows(tokens, heads), rows(keys, kv_heads), rows(keys, kv_heads)), types))
+        # keys and values whose scale changes along the sequence
+        k = k * torch.linspace(0.2, 2.0, keys, device=hip_device)[:, None].to(k.dtype)
+        v = v * torch.exp2(torch.arange(keys, device=hip_device) % 97 / 12.0 - 4.0)[:, None].to(v.dtype)
+        _check_attention(q, k, v, head_dim**-0.5, offset)
+
+
+def test_prompt_attention_zero_and_extreme_rows(hip_device):
+    """Zero value tiles, one-key rows and magnitudes far from 1 keep the accuracy (scales are powers of two)."""
+    g = torch.Generator(device=hip_device).manual_seed(3)
+    q, k, v = (torch.randn(1, h, 100, 64, generator=g, device=hip_device) for h in (2, 1, 1))
+    v[:, :, 32:64] = 0.0
+    for a, b in ((1.0, 1.0), (1e-20, 1e12), (1e15, 1e-18)):
+        _check_attention(q / a, k * a, v * b, 0.125, 0)
