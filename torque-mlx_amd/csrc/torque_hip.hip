@@ -713,6 +713,10 @@ __global__ __launch_bounds__(kBlock, 2) void decode_kernel(const DecodeArgs a) {
   const int hg = unit - lkv * a.n_hgroups;
   const int layer = lkv / a.kv_heads, kvh = lkv - layer * a.kv_heads;
   const int qh0 = kvh * a.group + hg * HG;
+  // Query heads of this head group: fewer than HG in the last one of a group
+  // that is no multiple of 4.  The missing heads' slots repeat the last head
+  // and are not stored.
+  const int heads = min(HG, a.group - hg * HG);
 
   // ---- tokens of this wavefront.  The sequence is cut into blocks of
   // STRIDE rows (one workgroup iteration) dealt out cyclically: split s takes
@@ -846,7 +850,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_kernel(const DecodeArgs a) {
   float qe[E], sg_first[E], sg_second[E];
   uint32_t qw[E];
   if (wave < HG) {
-    const int64_t qoff = (static_cast<int64_t>(layer) * a.query_heads + qh0 + wave) * D + lane * E;
+    const int64_t qoff = (static_cast<int64_t>(layer) * a.query_heads + qh0 + min(wave, heads - 1)) * D + lane * E;
     if constexpr (!QF16) {
       const uint32_t* q = static_cast<const uint32_t*>(a.q) + qoff;
 #pragma unroll
@@ -1300,7 +1304,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_kernel(const DecodeArgs a) {
   const int64_t qhg0 = static_cast<int64_t>(layer) * a.query_heads + qh0;
   if (a.n_splits == 1) {
     combine_waves();
-    if (wave < HG) {
+    if (wave < heads) {
       float f[kWavesPerBlock];
       const float M = wave_weights(wave, f);
       float l = 0.f;
@@ -1320,7 +1324,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_kernel(const DecodeArgs a) {
   // the current token's score per query head and its value per KV head.
   // Wavefront h < HG sums head h's row over the 4 wavefronts' partials
   // straight from LDS (no combining pass, no second barrier).
-  if (wave < HG) {
+  if (wave < heads) {
     float f[kWavesPerBlock];
     const float M = wave_weights(wave, f);
     float e[E];
@@ -1582,10 +1586,25 @@ __global__ __launch_bounds__(kStreamThreads) void stream_read_kernel(const uint4
 // ============================================================== host helpers
 
 
-int pick_hg(int group) {
-  if (group % 4 == 0) return 4;
-  if (group % 2 == 0) return 2;
-  return 1;
+// Query heads per work unit.  A unit reads its KV head's rows once, so groups
+// of 3 and more that are no multiple of 4 are cut into units of 4, the last
+// one with slots to spare (the matrix-core products cost the same whatever
+// the heads in them), where that saves enough rows (elements) to pay for the
+// longer set-up and combine of a 4-head unit.  Measured on MI355X against
+// units that divide the group: 8 KV heads, 3-bit rows at head_dim 128, 32768
+// tokens: groups of 3 25.2 -> 17.0 us, 5 38.6 -> 26.2, 6 32.7 -> 26.3, 7 48.3
+// -> 26.0; 16 x 8 heads at 64, 23236 tokens, groups of 3 124 -> 57; 10 M
+// elements saved 18.6 -> 16.1, but 4.2 M 9.3 -> 10.1 and 5.1 M (dense rows)
+// 7.5 -> 8.4.
+constexpr int64_t kMinSavedElements = int64_t(1) << 23;
+
+int head_groups(int group, int hg) { return (group + hg - 1) / hg; }
+int even_hg(int group) { return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }
+int pick_hg(int group, int64_t kv_units, int64_t seq_len, int head_dim) {
+  const int hg = even_hg(group);
+  if (hg == 4 || group < 3) return hg;
+  const int64_t saved = kv_units * (head_groups(group, hg) - head_groups(group, 4)) * seq_len * head_dim;
+  return saved >= kMinSavedElements ? 4 : hg;
 }
 
 // The split kernel a decode call runs: the float32 kernel (decode_kernel,
@@ -1773,8 +1792,8 @@ int fp32_tokens_per_iter(int fmt, int head_dim, int hg, int64_t seq_len, int64_t
 
 // Shapes the matrix-core split kernel takes: groups of 4 query heads with
 // 4-bit rows at head_dim 64 / 128 / 256 or 2-bit rows at head_dim 128.
-bool mx_shape(int fmt, int head_dim, int hg) {
-  return hg == 4 && ((fmt == 4 && (head_dim == 64 || head_dim == 128 || head_dim == 256)) ||
+bool mx_shape(int fmt, int head_dim, int group) {
+  return group % 4 == 0 && ((fmt == 4 && (head_dim == 64 || head_dim == 128 || head_dim == 256)) ||
                      (fmt == 2 && head_dim == 128));
 }
 
@@ -1810,10 +1829,10 @@ struct KernelChoice {
   SplitKernel kernel;
   int n_splits;
 };
-KernelChoice choose_kernel(int units, int64_t seq_len, int n_splits, int fmt, int head_dim, int hg, int flags,
+KernelChoice choose_kernel(int units, int64_t seq_len, int n_splits, int fmt, int head_dim, int group, int flags,
                            int num_cus) {
   if (n_splits <= 0 && one_split(seq_len, fmt, head_dim)) n_splits = 1;
-  if (mx_shape(fmt, head_dim, hg) && (flags & TQ_F32_PRODUCTS) == 0) {
+  if (mx_shape(fmt, head_dim, group) && (flags & TQ_F32_PRODUCTS) == 0) {
     const int ns = n_splits > 0 ? n_splits : default_splits(units, seq_len, num_cus, 1);
     const int64_t blocks = std::max<int64_t>(1, (seq_len + mx::kStride - 1) / mx::kStride);
     if ((flags & TQ_MATRIX_PRODUCTS) != 0 || blocks / std::min<int64_t>(blocks, ns) >= mx_min_blocks_per_split(head_dim))
@@ -1842,8 +1861,8 @@ int make_plan(int num_layers, int kv_heads, int query_heads, int64_t seq_len, in
                                     std::to_string(kv_heads));
   if (seq_len < 0) return fail(TQ_ERR_BAD_ARG, "seq_len must be non-negative");
   const int group = query_heads / kv_heads;
-  p->hg = pick_hg(group);
-  p->n_hgroups = group / p->hg;
+  p->hg = pick_hg(group, static_cast<int64_t>(num_layers) * kv_heads, seq_len, head_dim);
+  p->n_hgroups = head_groups(group, p->hg);
   // One launch holds at most 2^32 - 1 work-items: units x splits workgroups.
   const int64_t max_wg = ((int64_t(1) << 32) - 1) / kBlock;
   const int64_t units = static_cast<int64_t>(num_layers) * kv_heads * p->n_hgroups;
@@ -1852,7 +1871,7 @@ int make_plan(int num_layers, int kv_heads, int query_heads, int64_t seq_len, in
   p->units = static_cast<int>(units);
   if ((flags & TQ_F32_PRODUCTS) != 0 && (flags & TQ_MATRIX_PRODUCTS) != 0)
     return fail(TQ_ERR_BAD_ARG, "TQ_F32_PRODUCTS and TQ_MATRIX_PRODUCTS exclude each other");
-  const KernelChoice kc = choose_kernel(p->units, seq_len, n_splits, fmt, head_dim, p->hg, flags, device_cu_count());
+  const KernelChoice kc = choose_kernel(p->units, seq_len, n_splits, fmt, head_dim, group, flags, device_cu_count());
   p->kernel = kc.kernel;
   const int ns = kc.n_splits;
   if (ns > kMaxSplits) return fail(TQ_ERR_BAD_ARG, "n_splits must be at most " + std::to_string(kMaxSplits));
@@ -2675,10 +2694,10 @@ int tq_decode_default_splits(int num_layers, int kv_heads, int query_heads, int 
   if ((flags & TQ_F32_PRODUCTS) != 0 && (flags & TQ_MATRIX_PRODUCTS) != 0)
     return fail(TQ_ERR_BAD_ARG, "TQ_F32_PRODUCTS and TQ_MATRIX_PRODUCTS exclude each other");
   const int group = query_heads / kv_heads;
-  const int hg = pick_hg(group);
-  const int units = num_layers * kv_heads * (group / hg);
+  const int hg = pick_hg(group, static_cast<int64_t>(num_layers) * kv_heads, seq_len, head_dim);
+  const int units = num_layers * kv_heads * head_groups(group, hg);
   if (num_cus <= 0) num_cus = device_cu_count();
-  return choose_kernel(units, seq_len, 0, bits, head_dim, hg, flags, num_cus).n_splits;
+  return choose_kernel(units, seq_len, 0, bits, head_dim, group, flags, num_cus).n_splits;
 }
 
 const char* tq_decode_split_kernel(int num_layers, int kv_heads, int query_heads, int head_dim, int bits, int flags,
@@ -2698,11 +2717,11 @@ const char* tq_decode_split_kernel(int num_layers, int kv_heads, int query_heads
     return nullptr;
   }
   const int group = query_heads / kv_heads;
-  const int hg = pick_hg(group);
-  const int units = num_layers * kv_heads * (group / hg);
+  const int hg = pick_hg(group, static_cast<int64_t>(num_layers) * kv_heads, seq_len, head_dim);
+  const int units = num_layers * kv_heads * head_groups(group, hg);
   if (num_cus <= 0) num_cus = device_cu_count();
   static thread_local std::string name;
-  const KernelChoice kc = choose_kernel(units, seq_len, n_splits, bits, head_dim, hg, flags, num_cus);
+  const KernelChoice kc = choose_kernel(units, seq_len, n_splits, bits, head_dim, group, flags, num_cus);
   if (kc.kernel == SplitKernel::Mx)
     name = "decode_mx_kernel<" + std::to_string(head_dim) + "," + (query_dtype == TQ_F16 ? "true" : "false") +
            (bits == 4 ? ">" : "," + std::to_string(bits) + ">");
@@ -2719,8 +2738,8 @@ size_t tq_decode_workspace_bytes(int num_layers, int kv_heads, int query_heads, 
   if (num_layers <= 0 || kv_heads <= 0 || query_heads <= 0 || query_heads % kv_heads != 0) return 0;
   if (!valid_head_dim(head_dim)) return 0;
   const int group = query_heads / kv_heads;
-  const int hg = pick_hg(group);
-  const int units = num_layers * kv_heads * (group / hg);
+  // the fewest units a group is cut into, so the most splits
+  const int units = num_layers * kv_heads * head_groups(group, group >= 3 ? 4 : group);
   int ns = n_splits;
   // the larger of the two split kernels' defaults (two workgroups per CU, or
   // kMaxLoad where they are not all resident at once)
