@@ -47,3 +47,17 @@ def test_default_workspace_covers_every_plan():
 ])
 def test_workgroups_spread_over_the_cus(layers, kv, group, dim, bits, seq, most):
     assert _splits(layers, kv, group, dim, bits, 0, seq) == most
+
+
+@pytest.mark.parametrize("layers,kv,group,dim,bits,seq,default", [
+    (1, 4, 8, 128, 4, 30001, 64),  # units of 8 heads: 4 x 64 workgroups
+    (1, 8, 16, 128, 4, 32768, 16),
+    (24, 2, 8, 256, 4, 8192, 5),
+    (1, 4, 8, 128, 4, 8192, 64),  # too few blocks for the matrix kernel: units of 4 heads on the float32 kernel
+])
+def test_default_count_names_its_own_kernel(layers, kv, group, dim, bits, seq, default):
+    """The default count passed explicitly runs the kernel that the default runs."""
+    assert _splits(layers, kv, group, dim, bits, 0, seq) == default
+    name = lambda n: _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=layers, n_splits=n, num_cus=CUS)
+    assert name(0) == name(default)
+    assert ("mx" in name(0)) == (seq != 8192 or layers > 1)

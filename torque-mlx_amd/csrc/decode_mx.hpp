@@ -1,4 +1,4 @@
-// decode_mx_kernel -- split-K packed decode for groups of 4 query heads on the
+// decode_mx_kernel -- split-K packed decode for units of 4 or 8 query heads on the
 // gfx950 matrix cores with 16x16x32 float16 products (v_mfma_f32_16x16x32_f16).
 //
 // Included by torque_hip.hip (uses DecodeArgs, finish_row and tq_device.hpp).
@@ -53,6 +53,9 @@
 //   One product covers 16 tokens x 16 dims; the output of head h is row h +
 //   row 4 + h (lane groups 0 and 1, one permlane16 swap at the end).
 //
+//   Units of 8 heads fill the 16 columns and rows: hi splits of head h in
+//   column (row) h, lo splits in 8 + h.
+//
 // Tables: 256 entries x 8 bytes per stream, each entry replicated 32 times
 // so that lane l reads copy l % 32: entry e, copy c at byte e * 256 + c * 8
 // (64 KB per stream), which keeps 32 lanes' 8-byte reads on 32 distinct bank
@@ -88,24 +91,24 @@ constexpr int kTableBytes = 256 * kCopies * 8;
 constexpr int kPrefetch = 2;              // tiles whose loads are in flight ahead
 
 // LDS: the two tables, reused for the cross-wavefront reduction after the loop.
-template <int D>
+template <int D, int HG>
 struct Smem {
   static constexpr int kQbStride = D + 8;                // f16 elements per padded row (16-byte skew per row)
-  static constexpr int kQbBytes = 8 * kQbStride * 2;     // f16 query splits [8 cols][D]
-  static constexpr int kQBytes = 4 * D * 4;           // float32 scaled query [4][D]
+  static constexpr int kQbBytes = 2 * HG * kQbStride * 2;  // f16 query splits [2 HG cols][D]
+  static constexpr int kQBytes = HG * D * 4;          // float32 scaled query [HG][D]
   static constexpr int kCurBytes = 2 * D * 4 + 2 * D;  // append mode: s_cur [2][D] + codes [2][D]
   static constexpr int kMisc = 1024;
   static constexpr int kNW = waves_of<D>();
   static constexpr int kRS = D == 128 ? D + 6 : D < 128 ? D + 10 : D + 18;  // padded reduction row (floats)
-  static constexpr int kRedBytes = kNW * 4 * kRS * 4 + 2 * kNW * 4 * 4;      // rows, then (max, sum) per wave
+  static constexpr int kRedBytes = kNW * HG * kRS * 4 + 2 * kNW * HG * 4;      // rows, then (max, sum) per wave
   static constexpr int kQb = 2 * kTableBytes;
   static constexpr int kQ = kQb + kQbBytes;
   static constexpr int kCur = kQ + kQBytes;
   static constexpr int kMiscOff = kCur + kCurBytes;
   static constexpr int kSetup = kMiscOff + kMisc;
-  // The reduction sits beside the tables where the LDS holds both (head_dim
-  // 64 and 128), so each wavefront deposits its partial as soon as its own
-  // loop ends; at head_dim 256 it reuses the table area after a barrier.
+  // The reduction sits beside the tables where the LDS holds both (4 heads at
+  // head_dim 64 and 128), so each wavefront deposits its partial as soon as
+  // its own loop ends; otherwise it reuses the table area after a barrier.
   static constexpr bool kRedApart = kSetup + kRedBytes <= 160 * 1024;
   static constexpr int kRed = kRedApart ? kSetup : 0;
   static constexpr int kTotal = kRedApart ? kSetup + kRedBytes : kSetup;
@@ -235,12 +238,14 @@ __device__ __forceinline__ void write_tables2(uint8_t* smem, float cvec, int sh_
 
 }  // namespace mx
 
-template <int D, bool QF16, int BITS = 4>
+template <int D, bool QF16, int BITS, int HG>
 __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
     amdgpu_waves_per_eu(mx::waves_of<D>() / 4, mx::waves_of<D>() / 4))) void decode_mx_kernel(
     const DecodeArgs a) {
   using namespace mx;
   static_assert(D == 64 || D == 128 || D == 256, "head_dim 64, 128 or 256");
+  static_assert(HG == 4 || HG == 8, "4 or 8 query heads per unit");
+  constexpr bool H8 = HG == 8;
   static_assert(BITS == 4 || (BITS == 2 && D == 128), "4-bit rows, or 2-bit rows at head_dim 128");
   constexpr bool B2 = BITS == 2;      // 2-bit rows: 16-byte table entries, one per code byte
   constexpr int ROW = D * BITS / 8;   // packed bytes per row
@@ -259,14 +264,14 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
   constexpr int KBH = KB / NH;        // key bytes (lookups) per half
   constexpr int NSH = NS / NH;        // score products per half
   constexpr int NVH = NV / NH;        // value products per half
-  using L = Smem<D>;
+  using L = Smem<D, HG>;
 
   __shared__ __align__(16) uint8_t smem[L::kTotal];
-  uint16_t* s_qb = reinterpret_cast<uint16_t*>(smem + L::kQb);  // [8][D] f16 bits
-  float* s_q = reinterpret_cast<float*>(smem + L::kQ);           // [4][D]
+  uint16_t* s_qb = reinterpret_cast<uint16_t*>(smem + L::kQb);  // [2 HG][D] f16 bits
+  float* s_q = reinterpret_cast<float*>(smem + L::kQ);           // [HG][D]
   float* s_cur = reinterpret_cast<float*>(smem + L::kCur);       // [2][D]
   uint8_t* s_codes = smem + L::kCur + 2 * D * 4;                 // [2][D]
-  float* s_misc = reinterpret_cast<float*>(smem + L::kMiscOff);  // [0..3] score scale per head, [4] output scale
+  float* s_misc = reinterpret_cast<float*>(smem + L::kMiscOff);  // [0..HG-1] score scale per head, [HG] output scale
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: row ranges and resources stay scalar
@@ -274,9 +279,9 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
 
   // ---- work item: grid (split, head group, layer x KV head), so no
   // division is needed; the query heads of (lkv, hg) start at lkv * group +
-  // 4 hg of the [L * Hq] rows.
+  // HG hg of the [L * Hq] rows.
   const int split = blockIdx.x, hg = blockIdx.y, lkv = blockIdx.z;
-  const int64_t qhg0 = static_cast<int64_t>(lkv) * a.group + hg * 4;
+  const int64_t qhg0 = static_cast<int64_t>(lkv) * a.group + hg * HG;
 
   // Rows: blocks of kStride rows dealt out cyclically over the splits (split
   // s takes blocks s, s + n, s + 2n, ...), each block cut into
@@ -363,14 +368,19 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
 #pragma unroll
     for (int k = 0; k < kLevels; ++k) bnd[k] = b[k];
   }
-  float qe[E], sg_first[E], sg_second[E];
+  // wavefronts 0..3 prepare heads w and, in units of 8, w + 4
+  float qe[HG / 4][E], sg_first[E], sg_second[E];
   if (wave < 4) {
-    const int64_t qoff = (qhg0 + wave) * D + lane * E;
 #pragma unroll
-    for (int i = 0; i < E; ++i)
-      qe[i] = QF16 ? __half2float(static_cast<const __half*>(a.q)[qoff + i]) : static_cast<const float*>(a.q)[qoff + i];
+    for (int hh = 0; hh < HG / 4; ++hh) {
+      const int64_t qoff = (qhg0 + wave + 4 * hh) * D + lane * E;
+#pragma unroll
+      for (int i = 0; i < E; ++i)
+        qe[hh][i] =
+            QF16 ? __half2float(static_cast<const __half*>(a.q)[qoff + i]) : static_cast<const float*>(a.q)[qoff + i];
+    }
   }
-  if ((wave < 4 && (a.rotate_query || a.inverse_output)) || appender) {
+  if ((wave < HG && (a.rotate_query || a.inverse_output)) || appender) {
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       sg_first[i] = a.signs_right[lane * E + i];
@@ -412,7 +422,7 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
     else
       write_tables<NW - 4>(smem, cvec, sh_k, sh_v, wave - 4, lane);
   }
-  if (wave == 4 && lane == 0) s_misc[4] = ldexpf(1.f, -(sh_v + 7));  // weights carry 2^7, values 2^sh_v
+  if (wave == 4 && lane == 0) s_misc[HG] = ldexpf(1.f, -(sh_v + 7));  // weights carry 2^7, values 2^sh_v
 
   // ---- append mode: rotate (as on append) and quantize the new token.
   if (appender) {
@@ -429,25 +439,29 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
   // softmax scale and log2(e) folded in (scores come out in log2 units), then
   // the exact f16 split of q * 2^shift.
   if (wave < 4) {
-    if (a.rotate_query) wave_rotate_signs<D>(qe, sg_first, sg_second, a.sqrt_d);
-    float mxq = 0.f;
 #pragma unroll
-    for (int i = 0; i < E; ++i) {
-      qe[i] *= a.q_scale;
-      s_q[wave * D + lane * E + i] = qe[i];
-      mxq = fmaxf(mxq, fabsf(qe[i]));
-    }
-    mxq = group_reduce<kWave, OpMax>(mxq);
-    const int sh_q = scale_shift(mxq);
+    for (int hh = 0; hh < HG / 4; ++hh) {
+      const int head = wave + 4 * hh;
+      if (a.rotate_query) wave_rotate_signs<D>(qe[hh], sg_first, sg_second, a.sqrt_d);
+      float mxq = 0.f;
 #pragma unroll
-    for (int i = 0; i < E; ++i) {
-      const float x = ldexpf(qe[i], sh_q);
-      const _Float16 h = static_cast<_Float16>(x);
-      const _Float16 l = static_cast<_Float16>(x - static_cast<float>(h));
-      s_qb[wave * L::kQbStride + lane * E + i] = __builtin_bit_cast(uint16_t, h);
-      s_qb[(4 + wave) * L::kQbStride + lane * E + i] = __builtin_bit_cast(uint16_t, l);
+      for (int i = 0; i < E; ++i) {
+        qe[hh][i] *= a.q_scale;
+        s_q[head * D + lane * E + i] = qe[hh][i];
+        mxq = fmaxf(mxq, fabsf(qe[hh][i]));
+      }
+      mxq = group_reduce<kWave, OpMax>(mxq);
+      const int sh_q = scale_shift(mxq);
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        const float x = ldexpf(qe[hh][i], sh_q);
+        const _Float16 h = static_cast<_Float16>(x);
+        const _Float16 l = static_cast<_Float16>(x - static_cast<float>(h));
+        s_qb[head * L::kQbStride + lane * E + i] = __builtin_bit_cast(uint16_t, h);
+        s_qb[(HG + head) * L::kQbStride + lane * E + i] = __builtin_bit_cast(uint16_t, l);
+      }
+      if (lane == 0) s_misc[head] = ldexpf(1.f, -(sh_q + sh_k));  // raw score -> log2 units
     }
-    if (lane == 0) s_misc[wave] = ldexpf(1.f, -(sh_q + sh_k));  // raw score -> log2 units
   }
   if (wave >= 4) prefetch();
   // the set-up exchanges data through LDS only: the barrier leaves the
@@ -467,9 +481,9 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
   uint32_t qd[D / 8];  // f16 pairs of this lane's D / 4 dims
 #pragma unroll
   for (int i = 0; i < D / 8; ++i)
-    qd[i] = n < 8 ? reinterpret_cast<const uint32_t*>(s_qb + n * L::kQbStride + g * (D / 4))[i] : 0u;
-  const float score_scale = s_misc[n & 3];
-  const float out_scale = s_misc[4];
+    qd[i] = n < 2 * HG ? reinterpret_cast<const uint32_t*>(s_qb + n * L::kQbStride + g * (D / 4))[i] : 0u;
+  const float score_scale = s_misc[n & (HG - 1)];
+  const float out_scale = s_misc[HG];
 
   // table bases (offsets into smem): copy lane % 32 of 8-byte entries
   // (4-bit) or lane % 16 of 16-byte entries (2-bit), key table at 0, value
@@ -485,7 +499,8 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
   float m_lane = -INFINITY;
   float bias = INFINITY;  // +inf forces a maximum on the first tile
   float l_lane = 0.f;
-  const int kk = (lane >> 2) & 3;  // this lane's token within its lane group's 4
+  // this lane's token within its lane group's 4 (in units of 8: its first of two)
+  const int kk = H8 ? (n >> 3) * 2 : (lane >> 2) & 3;
   f32x4v acc[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) acc[j] = f32x4v{0.f, 0.f, 0.f, 0.f};
@@ -634,6 +649,64 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
     return as_f16x8(static_cast<uint32_t>(a0), static_cast<uint32_t>(a1), static_cast<uint32_t>(a2),
                     static_cast<uint32_t>(a3));
   };
+  // The same in units of 8: columns h and 8 + h hold head h's hi and lo query
+  // splits, so after a row_ror:8 add lanes n and n + 8 both hold head n % 8's
+  // scores of 4 tokens; lanes n < 8 work on tokens 0 and 1, the others on 2
+  // and 3, two exponentials to a lane.  Weight rows h are the hi splits, 8 +
+  // h the lo splits: the other half's pair is one row_ror:8 move.
+  auto softmax8 = [&](const f32x4v& ds, int k) {
+    float s4[4];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) s4[rr] = ds[rr] + dpp_move<kDppRor8>(ds[rr]);
+    const bool low = n < 8;
+    float sc[2] = {low ? s4[0] : s4[2], low ? s4[1] : s4[3]};
+    const int row0 = tile_row(k);
+    const bool full = row0 + kTile <= t1;  // wavefront-uniform
+    const bool valid[2] = {full || row0 + 4 * g + kk < t1, full || row0 + 4 * g + kk + 1 < t1};
+    float z[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      z[i] = fmaf(sc[i], score_scale, bias);
+      if (!full) z[i] = valid[i] ? z[i] : -INFINITY;
+    }
+    if (__builtin_amdgcn_ballot_w64(fmaxf(z[0], z[1]) > kRescaleThreshold + kWeightExp) != 0) {
+      float mx = fmaxf(valid[0] ? sc[0] * score_scale : -INFINITY, valid[1] ? sc[1] * score_scale : -INFINITY);
+      mx = strided_reduce<8, OpMax>(mx);
+      float alpha = 1.f;
+      if (mx > m_lane + kRescaleThreshold) {
+        alpha = fast_exp2(m_lane - mx);  // 0 before the first maximum
+        m_lane = mx;
+      }
+      l_lane *= alpha;
+      bias = kWeightExp - m_lane;
+      // register rr of lane group g holds head 4 (g % 2) + rr
+      f32x4v al;
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) al[rr] = __shfl(alpha, 4 * (g & 1) + rr);
+#pragma unroll
+      for (int j = 0; j < NV; ++j) acc[j] *= al;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) z[i] = valid[i] ? fmaf(sc[i], score_scale, bias) : -INFINITY;
+    }
+    int whi[2], wlo[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float p = fast_exp2(z[i]);  // p * 2^7
+      l_lane += p;
+      const float ph = __uint_as_float(__float_as_uint(p) & 0xffffe000u);
+      whi[i] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(ph, ph));
+      wlo[i] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(p - ph, p - ph));
+    }
+    // lanes 8..15 (banks 2, 3) take the lo pairs of lanes 0..7 for tokens 0
+    // and 1, lanes 0..7 the hi pairs of lanes 8..15 for tokens 2 and 3
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      w[i] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(whi[i], wlo[i], kDppRor8, 0xf, 0xc, false));
+      w[2 + i] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(wlo[i], whi[i], kDppRor8, 0xf, 0x3, false));
+    }
+    return as_f16x8(w[0], w[1], w[2], w[3]);
+  };
   auto value_products = [&](const f16x8& Aw, int h) {
 #pragma unroll
     for (int j = 0; j < NVH; ++j) {
@@ -666,7 +739,11 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
         scores(ds, h);
       }
       value_lookups(ring[j], 0);
-      const f16x8 Aw = softmax(ds, kq[j]);
+      f16x8 Aw;
+      if constexpr (H8)
+        Aw = softmax8(ds, kq[j]);
+      else
+        Aw = softmax(ds, kq[j]);
       value_products(Aw, 0);
 #pragma unroll
       for (int h = 1; h < NH; ++h) {
@@ -680,16 +757,16 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
     }
   }
 
-  // ---- combine: rows h and 4 + h (lane groups 0 and 1), then the
+  // ---- combine: rows h and HG + h (lane groups 0 and 1; 0, 1 and 2, 3), then the
   // wavefronts.  Lane n of group 0 holds head rr's output at dims of column n.
   if constexpr (!L::kRedApart) __syncthreads();  // the tables are dead: reuse their space
-  // s_red: [NW x 4 heads] rows of RS floats; dim d of a row sits at
+  // s_red: [NW x HG heads] rows of RS floats; dim d of a row sits at
   // d + 4 (d / 64), and RS = 2 (mod 4) and above that, so that the 32 lanes writing one
   // register pair (16 dims x 2 rows) hit 32 distinct banks
   constexpr int RS = L::kRS;
   float* s_red = reinterpret_cast<float*>(smem + L::kRed);
-  float* s_mw = reinterpret_cast<float*>(smem + L::kRed + NW * 4 * RS * 4);  // [NW][4]
-  float* s_lw = s_mw + NW * 4;                                       // [NW][4]
+  float* s_mw = reinterpret_cast<float*>(smem + L::kRed + NW * HG * RS * 4);  // [NW][HG]
+  float* s_lw = s_mw + NW * HG;                                      // [NW][HG]
   auto red_pos = [](int d) { return d + 4 * (d >> 6); };
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -700,15 +777,22 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
       // rows h (hi weights) and 4 + h (lo weights) of head h are lane groups
       // 0 and 1; one permlane16 swap sums two registers: group 0 receives
       // head 2pr's sum, group 1 head 2pr + 1's
-      const LanePair r = permlane_swap<16>(acc[j][2 * pr], acc[j][2 * pr + 1]);
-      if (g < 2) s_red[(wave * 4 + 2 * pr + g) * RS + red_pos(dim)] = r.first + r.second;
+      // (units of 8: rows h and 8 + h, lane groups g and g + 2 of heads 4 (g %
+      // 2) + register, by a permlane32 swap)
+      if constexpr (H8) {
+        const LanePair r = permlane_swap<32>(acc[j][2 * pr], acc[j][2 * pr + 1]);
+        s_red[(wave * HG + 4 * (g & 1) + 2 * pr + (g >> 1)) * RS + red_pos(dim)] = r.first + r.second;
+      } else {
+        const LanePair r = permlane_swap<16>(acc[j][2 * pr], acc[j][2 * pr + 1]);
+        if (g < 2) s_red[(wave * HG + 2 * pr + g) * RS + red_pos(dim)] = r.first + r.second;
+      }
     }
   }
   {
-    const float lw = strided_reduce<4, OpSum>(l_lane) * (1.f / 128.f);  // head lane % 4
-    if (lane < 4) {
-      s_mw[wave * 4 + lane] = m_lane;
-      s_lw[wave * 4 + lane] = lw;
+    const float lw = strided_reduce<HG, OpSum>(l_lane) * (1.f / 128.f);  // head lane % HG
+    if (lane < HG) {
+      s_mw[wave * HG + lane] = m_lane;
+      s_lw[wave * HG + lane] = lw;
     }
   }
   lds_barrier();  // the wavefronts' partials meet in LDS
@@ -716,23 +800,23 @@ __global__ __launch_bounds__(mx::threads_of<D>()) __attribute__((
   auto wave_weights = [&](int h, float (&f)[NW]) {
     float M = s_mw[h];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) M = fmaxf(M, s_mw[w * 4 + h]);
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, s_mw[w * HG + h]);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) f[w] = s_mw[w * 4 + h] == -INFINITY ? 0.f : fast_exp2(s_mw[w * 4 + h] - M);
+    for (int w = 0; w < NW; ++w) f[w] = s_mw[w * HG + h] == -INFINITY ? 0.f : fast_exp2(s_mw[w * HG + h] - M);
     return M;
   };
-  if (wave < 4) {
+  if (wave < HG) {
     float f[NW];
     const float M = wave_weights(wave, f);
     float l = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) l = fmaf(s_lw[w * 4 + wave], f[w], l);
+    for (int w = 0; w < NW; ++w) l = fmaf(s_lw[w * HG + wave], f[w], l);
     float e[E];
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       float v = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) v = fmaf(s_red[(w * 4 + wave) * RS + red_pos(lane * E + i)], f[w], v);
+      for (int w = 0; w < NW; ++w) v = fmaf(s_red[(w * HG + wave) * RS + red_pos(lane * E + i)], f[w], v);
       e[i] = v * out_scale;
     }
     if (a.n_splits == 1) {

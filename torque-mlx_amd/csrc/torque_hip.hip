@@ -1810,8 +1810,7 @@ int mx_min_blocks_per_split(int head_dim) { return head_dim == 256 ? 8 : 4; }
 // group reads them in 8 iterations at most and finishes its rows itself, so
 // the call is one launch.  Measured on MI355X (one decode on the GPU, then
 // with its Python call): 256 tokens x 8 heads at head_dim 128 6.0 / 8.5 us
-// against 7.4 / 11.4 in 2 splits, 512 tokens 7.8 / 8.6 against 7.3 / 11.6 (in
-// groups of 4, on the matrix kernel, 7.0 / 8.5 against 7.8 / 11.6), 768
+// against 7.4 / 11.4 in 2 splits, 512 tokens 7.8 / 8.6 against 7.3 / 11.6, 768
 // tokens 9.9 / 9.9 against 7.5 / 11.5; at head_dim 256 256 tokens 8.9 / 9.0
 // against 9.2 / 11.3, 384 tokens 11.2 / 11.2 against 9.3 / 11.4; at head_dim
 // 64 512 tokens 6.5 / 8.6 against 7.3 / 11.2.
@@ -1823,31 +1822,56 @@ bool one_split(int64_t seq_len, int fmt, int head_dim) {
   return packed && seq_len <= std::min(kShortTokens, kShortBlocks * decode_block_rows(fmt, head_dim));
 }
 
-// Split kernel and split count of a decode over `units` work units with
-// decode `flags` (n_splits <= 0: the default count for the chosen kernel).
+// Split kernel, split count and heads per unit of a decode over kv_units
+// (layers x KV heads) with decode `flags` (n_splits <= 0: the default count
+// for the chosen kernel).
 struct KernelChoice {
   SplitKernel kernel;
   int n_splits;
+  int hg;  // query heads per unit
 };
-KernelChoice choose_kernel(int units, int64_t seq_len, int n_splits, int fmt, int head_dim, int group, int flags,
+KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int fmt, int head_dim, int group, int flags,
                            int num_cus) {
-  if (n_splits <= 0 && one_split(seq_len, fmt, head_dim)) n_splits = 1;
-  if (mx_shape(fmt, head_dim, group) && (flags & TQ_F32_PRODUCTS) == 0) {
-    const int ns = n_splits > 0 ? n_splits : default_splits(units, seq_len, num_cus, 1);
-    const int64_t blocks = std::max<int64_t>(1, (seq_len + mx::kStride - 1) / mx::kStride);
-    if ((flags & TQ_MATRIX_PRODUCTS) != 0 || blocks / std::min<int64_t>(blocks, ns) >= mx_min_blocks_per_split(head_dim))
-      return {SplitKernel::Mx, ns};
-  }
-  if (n_splits > 0) return {SplitKernel::Fp32, n_splits};
   if (num_cus <= 0) num_cus = 256;
+  const int hg = pick_hg(group, kv_units, seq_len, head_dim);
+  const int units = static_cast<int>(kv_units * head_groups(group, hg));
+  const bool forced = (flags & TQ_MATRIX_PRODUCTS) != 0;
+  if (n_splits <= 0 && one_split(seq_len, fmt, head_dim)) {
+    if (!forced) return {SplitKernel::Fp32, 1, hg};
+    n_splits = 1;
+  }
+  if (mx_shape(fmt, head_dim, group) && (flags & TQ_F32_PRODUCTS) == 0) {
+    const int64_t blocks = std::max<int64_t>(1, (seq_len + mx::kStride - 1) / mx::kStride);
+    const int min_blocks = mx_min_blocks_per_split(head_dim);
+    const int ns4 = default_splits(units, seq_len, num_cus, 1);
+    const int ns = n_splits > 0 ? n_splits : ns4;
+    const bool runs = forced || blocks / std::min<int64_t>(blocks, ns) >= min_blocks;
+    // Units of 8 heads where units of 4 would run: one read of the rows and
+    // one lookup of every code for 8 heads, in products whose columns 4 heads
+    // fill by half.  Measured on MI355X, units of 4 -> 8: 4 KV heads x 30001
+    // 4-bit tokens at head_dim 128 13.6 -> 11.6 us, 8 x 32768 in groups of 16
+    // 28.8 -> 19.6, 12 layers x 8 x 8192 45.5 -> 34.2, 2 x 131072 at 256 31.5
+    // -> 23.8, 24 layers x 2 x 8192 at 256 59.7 -> 33.4.  An explicit count
+    // has to give more than half of the CUs a workgroup.
+    if (group % 8 == 0) {
+      const int ns8 = default_splits(units / 2, seq_len, num_cus, 1);
+      if (n_splits <= 0 || n_splits == ns8) {
+        if (forced || blocks / std::min<int64_t>(blocks, ns4) >= min_blocks) return {SplitKernel::Mx, ns8, 8};
+      } else if (forced || (runs && static_cast<int64_t>(units / 2) * n_splits > num_cus / 2)) {
+        return {SplitKernel::Mx, n_splits, 8};
+      }
+    }
+    if (runs) return {SplitKernel::Mx, ns, hg};
+  }
+  if (n_splits > 0) return {SplitKernel::Fp32, n_splits, hg};
   const int ns0 = default_splits(units, seq_len, num_cus, 2);
   // one split per kMinTokensPerSplit tokens at most, as in default_splits
   const int64_t by_len = (seq_len + kMinTokensPerSplit - 1) / kMinTokensPerSplit;
-  if (ns0 >= by_len) return {SplitKernel::Fp32, ns0};
+  if (ns0 >= by_len) return {SplitKernel::Fp32, ns0, hg};
   const bool packed = fmt == 2 || fmt == 3 || fmt == 4;
   const int64_t rows = decode_block_rows(packed ? fmt : 16, head_dim);  // dense rows: one plan for both types
   const int ns = balanced_splits(units, ns0, (seq_len + rows - 1) / rows, num_cus);
-  return {SplitKernel::Fp32, static_cast<int>(std::min<int64_t>(ns, by_len))};
+  return {SplitKernel::Fp32, static_cast<int>(std::min<int64_t>(ns, by_len)), hg};
 }
 
 // Fills the split plan of a decode call over `fmt` rows (see
@@ -1861,18 +1885,22 @@ int make_plan(int num_layers, int kv_heads, int query_heads, int64_t seq_len, in
                                     std::to_string(kv_heads));
   if (seq_len < 0) return fail(TQ_ERR_BAD_ARG, "seq_len must be non-negative");
   const int group = query_heads / kv_heads;
-  p->hg = pick_hg(group, static_cast<int64_t>(num_layers) * kv_heads, seq_len, head_dim);
+  const int64_t kv_units = static_cast<int64_t>(num_layers) * kv_heads;
+  p->hg = pick_hg(group, kv_units, seq_len, head_dim);
   p->n_hgroups = head_groups(group, p->hg);
   // One launch holds at most 2^32 - 1 work-items: units x splits workgroups.
   const int64_t max_wg = ((int64_t(1) << 32) - 1) / kBlock;
-  const int64_t units = static_cast<int64_t>(num_layers) * kv_heads * p->n_hgroups;
+  int64_t units = kv_units * p->n_hgroups;
   if (units > max_wg)
     return fail(TQ_ERR_BAD_ARG, "num_layers x kv_heads x head groups exceeds one launch; decode fewer layers per call");
-  p->units = static_cast<int>(units);
   if ((flags & TQ_F32_PRODUCTS) != 0 && (flags & TQ_MATRIX_PRODUCTS) != 0)
     return fail(TQ_ERR_BAD_ARG, "TQ_F32_PRODUCTS and TQ_MATRIX_PRODUCTS exclude each other");
-  const KernelChoice kc = choose_kernel(p->units, seq_len, n_splits, fmt, head_dim, group, flags, device_cu_count());
+  const KernelChoice kc = choose_kernel(kv_units, seq_len, n_splits, fmt, head_dim, group, flags, device_cu_count());
   p->kernel = kc.kernel;
+  p->hg = kc.hg;
+  p->n_hgroups = head_groups(group, p->hg);
+  units = kv_units * p->n_hgroups;
+  p->units = static_cast<int>(units);
   const int ns = kc.n_splits;
   if (ns > kMaxSplits) return fail(TQ_ERR_BAD_ARG, "n_splits must be at most " + std::to_string(kMaxSplits));
   p->tokens_per_iter = p->kernel == SplitKernel::Mx
@@ -1971,21 +1999,24 @@ struct ProfileEvents {
 int launch_merge(const MergeArgs& m, int num_layers, int query_heads, int head_dim, hipStream_t stream,
                  bool profiled, const ProfileEvents* caller_events);
 
-template <int D, bool QF16, int BITS>
+template <int D, bool QF16, int BITS, int HG>
 void launch_mx_t(const DecodeArgs& a, dim3 grid, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (start != nullptr || stop != nullptr)
-    hipExtLaunchKernelGGL((decode_mx_kernel<D, QF16, BITS>), grid, dim3(mx::threads_of<D>()), 0, stream, start,
+    hipExtLaunchKernelGGL((decode_mx_kernel<D, QF16, BITS, HG>), grid, dim3(mx::threads_of<D>()), 0, stream, start,
                           stop, 0, a);
   else
-    hipLaunchKernelGGL((decode_mx_kernel<D, QF16, BITS>), grid, dim3(mx::threads_of<D>()), 0, stream, a);
+    hipLaunchKernelGGL((decode_mx_kernel<D, QF16, BITS, HG>), grid, dim3(mx::threads_of<D>()), 0, stream, a);
 }
 
 template <int D, int BITS>
 void launch_mx_d(const DecodeArgs& a, dim3 grid, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+  const bool eight = a.n_hgroups * 8 == a.group;
   if (a.q_f16)
-    launch_mx_t<D, true, BITS>(a, grid, stream, start, stop);
+    eight ? launch_mx_t<D, true, BITS, 8>(a, grid, stream, start, stop)
+          : launch_mx_t<D, true, BITS, 4>(a, grid, stream, start, stop);
   else
-    launch_mx_t<D, false, BITS>(a, grid, stream, start, stop);
+    eight ? launch_mx_t<D, false, BITS, 8>(a, grid, stream, start, stop)
+          : launch_mx_t<D, false, BITS, 4>(a, grid, stream, start, stop);
 }
 
 // Grid (split, head group, layer x KV head) of decode_mx_kernel.
@@ -2694,10 +2725,9 @@ int tq_decode_default_splits(int num_layers, int kv_heads, int query_heads, int 
   if ((flags & TQ_F32_PRODUCTS) != 0 && (flags & TQ_MATRIX_PRODUCTS) != 0)
     return fail(TQ_ERR_BAD_ARG, "TQ_F32_PRODUCTS and TQ_MATRIX_PRODUCTS exclude each other");
   const int group = query_heads / kv_heads;
-  const int hg = pick_hg(group, static_cast<int64_t>(num_layers) * kv_heads, seq_len, head_dim);
-  const int units = num_layers * kv_heads * head_groups(group, hg);
   if (num_cus <= 0) num_cus = device_cu_count();
-  return choose_kernel(units, seq_len, 0, bits, head_dim, group, flags, num_cus).n_splits;
+  const int64_t kv_units = static_cast<int64_t>(num_layers) * kv_heads;
+  return choose_kernel(kv_units, seq_len, 0, bits, head_dim, group, flags, num_cus).n_splits;
 }
 
 const char* tq_decode_split_kernel(int num_layers, int kv_heads, int query_heads, int head_dim, int bits, int flags,
@@ -2717,19 +2747,18 @@ const char* tq_decode_split_kernel(int num_layers, int kv_heads, int query_heads
     return nullptr;
   }
   const int group = query_heads / kv_heads;
-  const int hg = pick_hg(group, static_cast<int64_t>(num_layers) * kv_heads, seq_len, head_dim);
-  const int units = num_layers * kv_heads * head_groups(group, hg);
   if (num_cus <= 0) num_cus = device_cu_count();
+  const int64_t kv_units = static_cast<int64_t>(num_layers) * kv_heads;
   static thread_local std::string name;
-  const KernelChoice kc = choose_kernel(units, seq_len, n_splits, bits, head_dim, group, flags, num_cus);
+  const KernelChoice kc = choose_kernel(kv_units, seq_len, n_splits, bits, head_dim, group, flags, num_cus);
   if (kc.kernel == SplitKernel::Mx)
     name = "decode_mx_kernel<" + std::to_string(head_dim) + "," + (query_dtype == TQ_F16 ? "true" : "false") +
            (bits == 4 ? ">" : "," + std::to_string(bits) + ">");
-  else if (fp32_tokens_per_iter(bits, head_dim, hg, seq_len, kc.n_splits) == kWideTokensPerIter)
+  else if (fp32_tokens_per_iter(bits, head_dim, kc.hg, seq_len, kc.n_splits) == kWideTokensPerIter)
     name = "decode_kernel<PackedB4,256,4," + std::to_string(kWideTokensPerIter) + ">";
   else
     name = "decode_kernel<PackedB" + std::to_string(bits) + "," + std::to_string(head_dim) + "," +
-           std::to_string(hg) + ">";
+           std::to_string(kc.hg) + ">";
   return name.c_str();
 }
 
@@ -2790,7 +2819,7 @@ int tq_decode_noalloc(const void* query, int query_dtype, int num_layers, int qu
   if (rc) return rc;
   return decode_common(bits, query, query_dtype, num_layers, query_heads, kv_heads, head_dim, key_codes,
                        value_codes, capacity, seq_len, key_centroids, value_centroids, signs_left, signs_right, flags,
-                       current_keys, current_values, p.n_splits, ws, kScratchBytes, out, stream, nullptr, nullptr);
+                       current_keys, current_values, n_splits, ws, kScratchBytes, out, stream, nullptr, nullptr);
 }
 
 int tq_decode_scaled(const void* query, int query_dtype, int num_layers, int query_heads, int kv_heads, int head_dim,
