@@ -42,7 +42,7 @@ enum {
   TQ_ERR_LAUNCH = -3       /* HIP launch failure (Python: RuntimeError) */
 };
 
-enum { TQ_F32 = 0, TQ_F16 = 1, TQ_BF16 = 2 /* tq_rotary, tq_unrotate_gate, tq_prompt_attention only */ };
+enum { TQ_F32 = 0, TQ_F16 = 1, TQ_BF16 = 2 /* tq_rotary and tq_unrotate_gate only */ };
 
 /* tq_append / tq_quantize_dequantize flags (reference cache_mlx.py:52-54) */
 enum { TQ_ROTATE_KEYS = 1, TQ_ROTATE_VALUES = 2 };
@@ -326,22 +326,6 @@ int tq_unrotate_gate(const float* attn, int heads, int64_t tokens, int head_dim,
                      int64_t token_stride, const void* gate, int gate_dtype, int64_t gate_head_stride,
                      int64_t gate_token_stride, const float* signs_left, const float* signs_right, void* out,
                      int out_dtype, hipStream_t stream);
-
-/* Causal attention of a prompt chunk over dense keys and values (reference
- * qwen_mlx.py:838-853, the dense attention of a multi-token chunk): query row
- * i attends keys 0 .. offset + i (all num_keys at most).  query [query_heads,
- * tokens, head_dim], keys / values [kv_heads, num_keys, head_dim], each in its
- * own dtype (TQ_F32, TQ_F16, TQ_BF16) with element strides and unit stride
- * along head_dim; out contiguous float32 [query_heads, tokens, head_dim].
- * Products are exact float16 hi / lo splits summed in float32 (three of the
- * four cross terms): float32 accuracy.  The workspace, 16-byte aligned, holds
- * the split keys and values of this call; it needs no initialisation. */
-size_t tq_prompt_attention_workspace_bytes(int kv_heads, int64_t keys, int head_dim);
-int tq_prompt_attention(const void* query, int q_dtype, int query_heads, int64_t q_head_stride, int64_t q_token_stride,
-                        const void* keys, int k_dtype, int64_t k_head_stride, int64_t k_token_stride,
-                        const void* values, int v_dtype, int64_t v_head_stride, int64_t v_token_stride, int kv_heads,
-                        int64_t tokens, int64_t num_keys, int64_t offset, int head_dim, float scale, void* workspace,
-                        size_t workspace_bytes, float* out, hipStream_t stream);
 
 /* Measurement helper, no counterpart in the reference: streams `bytes` bytes
  * (a multiple of 16, 16-byte aligned) through nontemporal 16-byte loads,

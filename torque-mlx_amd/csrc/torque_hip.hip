@@ -1548,7 +1548,6 @@ __global__ __launch_bounds__(kBlock) void accumulate_kernel(const float* __restr
 
 
 #include "attention_layer.hpp"
-#include "prompt_attention.hpp"
 
 // ============================================================== measurement
 
@@ -2610,17 +2609,6 @@ int unpack_impl(const uint32_t* codes, int64_t groups, int64_t capacity, int64_t
   return with_d<UnpackBody>(head_dim, codes, groups, capacity, seq_len, bits, centroids, scales, out, stream);
 }
 
-template <int D>
-struct PromptBody {
-  static int run(const PromptArgs& a, unsigned groups, unsigned kv_heads, hipStream_t stream) {
-    hipLaunchKernelGGL(pack_kv_kernel<D>, dim3(a.tiles, kv_heads), dim3(kBlock), 0, stream, a);
-    int rc = launch_status("pack_kv_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(prompt_attention_kernel<D>, dim3(groups, kv_heads), dim3(kBlock), 0, stream, a);
-    return launch_status("prompt_attention_kernel");
-  }
-};
-
 }  // namespace
 
 // ============================================================== C ABI
@@ -3014,51 +3002,6 @@ int tq_unrotate_gate(const float* attn, int heads, int64_t tokens, int head_dim,
   else
     hipLaunchKernelGGL(unrotate_gate_kernel<256>, grid, dim3(kBlock), 0, stream, a);
   return launch_status("unrotate_gate_kernel");
-}
-
-size_t tq_prompt_attention_workspace_bytes(int kv_heads, int64_t keys, int head_dim) {
-  if (kv_heads <= 0 || keys <= 0 || !valid_head_dim(head_dim)) return 0;
-  const size_t tiles = static_cast<size_t>(kv_heads) * ((keys + prompt::kTileKeys - 1) / prompt::kTileKeys);
-  return tiles * prompt::tile_bytes(head_dim) + align256(tiles * sizeof(int2));
-}
-
-int tq_prompt_attention(const void* query, int q_dtype, int query_heads, int64_t q_head_stride, int64_t q_token_stride,
-                        const void* keys, int k_dtype, int64_t k_head_stride, int64_t k_token_stride,
-                        const void* values, int v_dtype, int64_t v_head_stride, int64_t v_token_stride, int kv_heads,
-                        int64_t tokens, int64_t num_keys, int64_t offset, int head_dim, float scale, void* workspace,
-                        size_t workspace_bytes, float* out, hipStream_t stream) {
-  const int rc = check_geometry(head_dim, 0);
-  if (rc) return rc;
-  if (query_heads <= 0 || kv_heads <= 0 || query_heads % kv_heads != 0)
-    return fail(TQ_ERR_BAD_ARG, "query_heads must be a positive multiple of kv_heads");
-  if (tokens < 0 || num_keys <= 0 || offset < 0) return fail(TQ_ERR_BAD_ARG, "bad attention extents");
-  for (int type : {q_dtype, k_dtype, v_dtype})
-    if (type < TQ_F32 || type > TQ_BF16) return fail(TQ_ERR_BAD_ARG, "dtypes must be F32, F16 or BF16");
-  if (tokens == 0) return TQ_OK;
-  if (!query || !keys || !values || !workspace || !out) return fail(TQ_ERR_BAD_ARG, "null pointer argument");
-  if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0)
-    return fail(TQ_ERR_BAD_ARG, "workspace and out must be 16-byte aligned");
-  if (workspace_bytes < tq_prompt_attention_workspace_bytes(kv_heads, num_keys, head_dim))
-    return fail(TQ_ERR_BAD_ARG, "workspace is smaller than tq_prompt_attention_workspace_bytes");
-  const int64_t tiles = (num_keys + prompt::kTileKeys - 1) / prompt::kTileKeys;
-  const int group = query_heads / kv_heads;
-  const int64_t groups = ((tokens + prompt::kRows - 1) / prompt::kRows * group + kWavesPerBlock - 1) / kWavesPerBlock;
-  if (tiles > (1 << 22) || groups > (1 << 22) || kv_heads > 65535)
-    return fail(TQ_ERR_BAD_ARG, "prompt attention exceeds one launch");
-  PromptArgs a{};
-  a.q = {query, q_dtype, query_heads, q_head_stride, q_token_stride};
-  a.k = {keys, k_dtype, kv_heads, k_head_stride, k_token_stride};
-  a.v = {values, v_dtype, kv_heads, v_head_stride, v_token_stride};
-  a.tokens = tokens;
-  a.keys = num_keys;
-  a.offset = offset;
-  a.scale = scale;
-  a.group = group;
-  a.tiles = static_cast<int>(tiles);
-  a.packed = static_cast<uint4*>(workspace);
-  a.shifts = reinterpret_cast<int2*>(static_cast<uint8_t*>(workspace) + kv_heads * tiles * prompt::tile_bytes(head_dim));
-  a.out = out;
-  return with_d<PromptBody>(head_dim, a, static_cast<unsigned>(groups), static_cast<unsigned>(kv_heads), stream);
 }
 
 int tq_stream_read(const void* data, size_t bytes, float* sink, int n_blocks, hipStream_t stream, hipEvent_t start,

@@ -28,7 +28,7 @@ TQ_ERR_LAUNCH = -3
 
 TQ_F32 = 0
 TQ_F16 = 1
-TQ_BF16 = 2  # tq_rotary, tq_unrotate_gate and tq_prompt_attention only
+TQ_BF16 = 2  # tq_rotary and tq_unrotate_gate only
 
 TQ_ROTATE_KEYS = 1
 TQ_ROTATE_VALUES = 2
@@ -102,11 +102,6 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         [_p, _p, _i, _i, _i, _i64, _i, _i64, _i64, _i64, _i64, _p, _p, _i, _i64, _i64, _i, _p, _p, _i, _p],
     ),
     "tq_unrotate_gate": (_i, [_p, _i, _i64, _i, _i64, _i64, _p, _i, _i64, _i64, _p, _p, _p, _i, _p]),
-    "tq_prompt_attention_workspace_bytes": (_sz, [_i, _i64, _i]),
-    "tq_prompt_attention": (
-        _i,
-        [_p, _i, _i, _i64, _i64, _p, _i, _i64, _i64, _p, _i, _i64, _i64, _i, _i64, _i64, _i64, _i, _f, _p, _sz, _p, _p],
-    ),
     "tq_stream_read": (_i, [_p, _sz, _p, _i, _p, _p, _p]),
 }
 
@@ -154,8 +149,7 @@ def check(rc: int) -> None:
     raise TorqueHIPError(message or f"libtorque_hip error {rc}")
 
 
-_NOT_STATUS = {"tq_abi_version", "tq_last_error", "tq_decode_workspace_bytes", "tq_decode_split_kernel",
-               "tq_prompt_attention_workspace_bytes"}
+_NOT_STATUS = {"tq_abi_version", "tq_last_error", "tq_decode_workspace_bytes", "tq_decode_split_kernel"}
 
 
 def call(name: str, *args) -> int:

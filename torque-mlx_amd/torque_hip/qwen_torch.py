@@ -310,39 +310,8 @@ def _unrotate_gate(attn_output: torch.Tensor, gate: torch.Tensor, *, rotation: R
     return (output * torch.sigmoid(gate.reshape(1, tokens, -1).float())).to(dtype)
 
 
-def _prompt_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
-    return (
-        q.dim() == k.dim() == v.dim() == 4
-        and q.shape[0] == k.shape[0] == 1
-        and k.shape == v.shape
-        and q.shape[3] == k.shape[3]
-        and q.shape[3] in (64, 128, 256)
-        and 0 not in (*q.shape, *k.shape)
-        and q.shape[1] % k.shape[1] == 0
-        and q.stride(3) == k.stride(3) == v.stride(3) == 1
-        and _plain(q, k, v)
-    )
-
-
-def _prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float, offset: int) -> torch.Tensor:
-    """``tq_prompt_attention`` of [1, Hq, L, D] queries over [1, Hkv, S, D] keys and values; float32 result."""
-    _, heads, tokens, dim = q.shape
-    kv_heads, keys = k.shape[1], k.shape[2]
-    nbytes = _lib.call("tq_prompt_attention_workspace_bytes", kv_heads, keys, dim)
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-    out = torch.empty((1, heads, tokens, dim), dtype=torch.float32, device=q.device)
-    _lib.call(
-        "tq_prompt_attention", q.data_ptr(), _TYPES[q.dtype], heads, q.stride(1), q.stride(2), k.data_ptr(), _TYPES[k.dtype],
-        k.stride(1), k.stride(2), v.data_ptr(), _TYPES[v.dtype], v.stride(1), v.stride(2), kv_heads, tokens, keys, offset, dim,
-        float(scale), workspace.data_ptr(), nbytes, out.data_ptr(), stream_handle(q.device),
-    )
-    return out
-
-
 def _dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float, offset: int) -> torch.Tensor:
     """Causal attention of L new queries at positions offset.. over all S cached keys, float32 math."""
-    if _prompt_kernel_takes(q, k, v):
-        return _prompt_attention(q, k, v, scale=scale, offset=offset)
     group = int(q.shape[1]) // int(k.shape[1])
     k = k.to(torch.float32).repeat_interleave(group, dim=1)
     v = v.to(torch.float32).repeat_interleave(group, dim=1)
