@@ -84,6 +84,21 @@ def test_gradients_and_transforms_keep_the_torch_operations(hip_device):
     assert gate.grad is not None and gate.grad.abs().sum() > 0
 
 
+def test_operands_of_another_device_keep_the_torch_operations(hip_device, monkeypatch):
+    """The library launches on the current device: tensors of another one go through torch, which guards its calls."""
+    from torque_hip import _lib
+    from torque_hip import qwen_torch as qt
+
+    q, k = torch.randn(1, 2, 3, 64, device=hip_device), torch.randn(1, 1, 3, 64, device=hip_device)
+    cos, sin = torch.randn(1, 3, 16, device=hip_device), torch.randn(1, 3, 16, device=hip_device)
+    assert qt._plain(q, k, cos, sin)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: hip_device.index + 1)
+    monkeypatch.setattr(_lib, "call", lambda *args: pytest.fail("launched on the current device"))
+    assert not qt._plain(q, k, cos, sin)
+    for y, x in zip(qt.apply_rotary(q, k, cos, sin), (q, k)):
+        assert torch.equal(y, _rotary_reference(x, cos, sin))
+
+
 def _check_attention(q, k, v, scale, offset, rows=slice(None)):
     """Against float64, as float32 attention.  A float32 score is a sum of D products, off by at most (D + 1) 2^-24 of
     its sum of magnitudes A however the products are grouped, and in fact by a few 2^-24; with 2 A 2^-22 allowed to a

@@ -230,8 +230,9 @@ _TYPES = {torch.float32: _lib.TQ_F32, torch.float16: _lib.TQ_F16, torch.bfloat16
 
 
 def _plain(*tensors: torch.Tensor) -> bool:
-    """Whether a kernel may read these tensors directly: ordinary tensors of one GPU and a type it takes, with no
-    gradient, transform, trace or dispatch mode to see the operations it stands for."""
+    """Whether a kernel may read these tensors directly: ordinary tensors of the current GPU (the library launches
+    there; torch's operations go to their tensors' own) and a type it takes, with no gradient, transform, trace or
+    dispatch mode to see the operations it stands for."""
     dev = tensors[0].device
     for t in tensors:
         if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
@@ -240,6 +241,7 @@ def _plain(*tensors: torch.Tensor) -> bool:
             return False
     return (
         dev.type == "cuda"
+        and dev.index == torch.cuda.current_device()
         and not torch.compiler.is_compiling()
         and not torch.jit.is_tracing()
         and torch._C._functorch.peek_interpreter_stack() is None
