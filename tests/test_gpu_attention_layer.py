@@ -84,6 +84,28 @@ def test_gradients_and_transforms_keep_the_torch_operations(hip_device):
     assert gate.grad is not None and gate.grad.abs().sum() > 0
 
 
+def test_rows_past_one_launch(hip_device):
+    """More rows than the 2^32 - 1 work-items of one launch hold at a wavefront each (2^26): a call is cut into several."""
+    from torque_hip import RotationSpec
+    from torque_hip import qwen_torch as qt
+
+    g = torch.Generator(device=hip_device).manual_seed(1)
+    tokens = 2**25 + 3
+    q, k = (torch.randn(1, 1, tokens, 2, generator=g, device=hip_device, dtype=torch.float16) for _ in range(2))
+    cos, sin = (torch.randn(1, tokens, 2, generator=g, device=hip_device, dtype=torch.float16) for _ in range(2))
+    for y, x in zip(qt.apply_rotary(q, k, cos, sin), (q, k)):
+        assert torch.equal(y, _rotary_reference(x, cos, sin))
+    del q, k, cos, sin, x, y
+    heads, tokens = 64, 2**20 + 1
+    attn = torch.randn(1, 1, tokens, 64, generator=g, device=hip_device).expand(1, heads, tokens, 64)
+    gate = torch.randn(1, tokens, 1, 64, generator=g, device=hip_device).expand(1, tokens, heads, 64)
+    rotation = RotationSpec.from_seed(64, 3)
+    one = qt._unrotate_gate(attn[:, :1], gate[:, :, :1], rotation=rotation, dtype=torch.bfloat16)
+    got = qt._unrotate_gate(attn, gate, rotation=rotation, dtype=torch.bfloat16).view(tokens, heads, 64)
+    for h in range(heads):
+        assert torch.equal(got[:, h], one[0])
+
+
 def test_operands_of_another_device_keep_the_torch_operations(hip_device, monkeypatch):
     """The library launches on the current device: tensors of another one go through torch, which guards its calls."""
     from torque_hip import _lib

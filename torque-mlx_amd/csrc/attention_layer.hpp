@@ -52,14 +52,15 @@ struct RotaryArgs {
   const void* sin;
   int table_type;
   int64_t cos_stride, sin_stride;
-  int tokens, head_dim, rotary_dim;
+  int64_t tokens, row0;  // row0: first row of this launch
+  int head_dim, rotary_dim;
 };
 
 // One wavefront per row of queries (then keys): x cos + rotate_half(x) sin on
 // the first rotary_dim dimensions, the rest copied.  At prompt sizes it reads
 // and writes each row once and is bound by memory.
 __global__ __launch_bounds__(kBlock) void rotary_kernel(const RotaryArgs a) {
-  int64_t row = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
+  int64_t row = a.row0 + static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
   const int64_t q_rows = static_cast<int64_t>(a.x[0].heads) * a.tokens;
   const int s = row >= q_rows;
   if (s) row -= q_rows;
@@ -87,7 +88,7 @@ struct GateArgs {
   RowView gate;
   void* out;          // contiguous [tokens, heads * D] of out_type
   int out_type;
-  int tokens;
+  int64_t tokens, row0;  // row0: first row of this launch
   const float* signs_left;
   const float* signs_right;
   float sqrt_d;
@@ -98,7 +99,7 @@ struct GateArgs {
 template <int D>
 __global__ __launch_bounds__(kBlock) void unrotate_gate_kernel(const GateArgs a) {
   constexpr int E = D / kWave;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
+  const int64_t row = a.row0 + static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
   if (row >= static_cast<int64_t>(a.attn.heads) * a.tokens) return;  // whole wavefront exits together
   const int64_t t = row / a.attn.heads, h = row - t * a.attn.heads;
   const int d0 = lane_id() * E;

@@ -2280,10 +2280,15 @@ int with_d(int head_dim, Args&&... args) {
   return fail(TQ_ERR_UNSUPPORTED, "Unsupported head dimension: " + std::to_string(head_dim));
 }
 
-// Workgroups per launch of the row kernels (fwht, append, unpack).  A HIP
-// launch holds at most 2^32 - 1 work-items; larger calls are cut into
-// launches of at most this many workgroups, in stream order.
+// Workgroups per launch of the row kernels (fwht, append, unpack, rotary,
+// gate).  A HIP launch holds at most 2^32 - 1 work-items; larger calls are cut
+// into launches of at most this many workgroups, in stream order.
 constexpr int64_t kMaxLaunchBlocks = int64_t(1) << 20;
+
+// Grid of one launch of a kernel with a wavefront per row, `rows` left to do.
+dim3 row_grid(int64_t rows) {
+  return dim3(static_cast<unsigned>(std::min((rows + kWavesPerBlock - 1) / kWavesPerBlock, kMaxLaunchBlocks)));
+}
 
 template <int D>
 struct FwhtBody {
@@ -2950,8 +2955,6 @@ int tq_rotary(const void* query, const void* key, int x_dtype, int query_heads, 
   const int64_t rows = (static_cast<int64_t>(query_heads) + key_heads) * tokens;
   if (rows == 0) return TQ_OK;
   if (!query || !key || !cos || !sin || !query_out || !key_out) return fail(TQ_ERR_BAD_ARG, "null pointer argument");
-  if (tokens > INT32_MAX || (rows + kWavesPerBlock - 1) / kWavesPerBlock > ((int64_t(1) << 32) - 1) / kBlock)
-    return fail(TQ_ERR_BAD_ARG, "heads x tokens exceeds one launch");
   RotaryArgs a{};
   a.x[0] = {query, x_dtype, query_heads, q_head_stride, q_token_stride};
   a.x[1] = {key, x_dtype, key_heads, k_head_stride, k_token_stride};
@@ -2963,12 +2966,15 @@ int tq_rotary(const void* query, const void* key, int x_dtype, int query_heads, 
   a.table_type = table_dtype;
   a.cos_stride = cos_stride;
   a.sin_stride = sin_stride;
-  a.tokens = static_cast<int>(tokens);
+  a.tokens = tokens;
   a.head_dim = head_dim;
   a.rotary_dim = rotary_dim;
-  const unsigned nblk = static_cast<unsigned>((rows + kWavesPerBlock - 1) / kWavesPerBlock);
-  hipLaunchKernelGGL(rotary_kernel, dim3(nblk), dim3(kBlock), 0, stream, a);
-  return launch_status("rotary_kernel");
+  for (a.row0 = 0; a.row0 < rows; a.row0 += kMaxLaunchBlocks * kWavesPerBlock) {
+    hipLaunchKernelGGL(rotary_kernel, row_grid(rows - a.row0), dim3(kBlock), 0, stream, a);
+    const int rc = launch_status("rotary_kernel");
+    if (rc) return rc;
+  }
+  return TQ_OK;
 }
 
 int tq_unrotate_gate(const float* attn, int heads, int64_t tokens, int head_dim, int64_t head_stride,
@@ -2983,25 +2989,27 @@ int tq_unrotate_gate(const float* attn, int heads, int64_t tokens, int head_dim,
   const int64_t rows = heads * tokens;
   if (rows == 0) return TQ_OK;
   if (!attn || !gate || !signs_left || !signs_right || !out) return fail(TQ_ERR_BAD_ARG, "null pointer argument");
-  if (tokens > INT32_MAX || (rows + kWavesPerBlock - 1) / kWavesPerBlock > ((int64_t(1) << 32) - 1) / kBlock)
-    return fail(TQ_ERR_BAD_ARG, "heads x tokens exceeds one launch");
   GateArgs a{};
   a.attn = {attn, kTypeF32, heads, head_stride, token_stride};
   a.gate = {gate, gate_dtype, heads, gate_head_stride, gate_token_stride};
   a.out = out;
   a.out_type = out_dtype;
-  a.tokens = static_cast<int>(tokens);
+  a.tokens = tokens;
   a.signs_left = signs_left;
   a.signs_right = signs_right;
   a.sqrt_d = sqrt_f32(head_dim);
-  const dim3 grid(static_cast<unsigned>((rows + kWavesPerBlock - 1) / kWavesPerBlock));
-  if (head_dim == 64)
-    hipLaunchKernelGGL(unrotate_gate_kernel<64>, grid, dim3(kBlock), 0, stream, a);
-  else if (head_dim == 128)
-    hipLaunchKernelGGL(unrotate_gate_kernel<128>, grid, dim3(kBlock), 0, stream, a);
-  else
-    hipLaunchKernelGGL(unrotate_gate_kernel<256>, grid, dim3(kBlock), 0, stream, a);
-  return launch_status("unrotate_gate_kernel");
+  for (a.row0 = 0; a.row0 < rows; a.row0 += kMaxLaunchBlocks * kWavesPerBlock) {
+    const dim3 grid = row_grid(rows - a.row0);
+    if (head_dim == 64)
+      hipLaunchKernelGGL(unrotate_gate_kernel<64>, grid, dim3(kBlock), 0, stream, a);
+    else if (head_dim == 128)
+      hipLaunchKernelGGL(unrotate_gate_kernel<128>, grid, dim3(kBlock), 0, stream, a);
+    else
+      hipLaunchKernelGGL(unrotate_gate_kernel<256>, grid, dim3(kBlock), 0, stream, a);
+    const int rc_launch = launch_status("unrotate_gate_kernel");
+    if (rc_launch) return rc_launch;
+  }
+  return TQ_OK;
 }
 
 int tq_stream_read(const void* data, size_t bytes, float* sink, int n_blocks, hipStream_t stream, hipEvent_t start,
