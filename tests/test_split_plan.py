@@ -61,3 +61,17 @@ def test_default_count_names_its_own_kernel(layers, kv, group, dim, bits, seq, d
     name = lambda n: _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=layers, n_splits=n, num_cus=CUS)
     assert name(0) == name(default)
     assert ("mx" in name(0)) == (seq != 8192 or layers > 1)
+
+
+@pytest.mark.parametrize("layers,kv,group,dim,bits", [
+    (24, 8, 4, 64, 4), (24, 8, 4, 128, 4), (24, 8, 4, 128, 2), (48, 4, 4, 128, 4), (12, 8, 8, 128, 4), (24, 8, 8, 64, 4), (24, 4, 16, 128, 2),
+])
+def test_one_split_of_many_units_keeps_the_matrix_kernel(layers, kv, group, dim, bits):
+    """Where the matrix kernel's own plan is one split of at least 4 blocks of 128 rows, a short sequence runs on it; with
+    fewer rows, or with units too few for one split each, on the float32 kernel."""
+    name = lambda seq, layers: _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=layers, n_splits=0, num_cus=CUS)
+    for seq in (385, 450, 512):
+        assert _splits(layers, kv, group, dim, bits, 0, seq) == 1
+        assert "mx" in name(seq, layers)
+        assert "mx" not in name(seq, 1)
+    assert "mx" not in name(384, layers)

@@ -1835,14 +1835,18 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
   const int hg = pick_hg(group, kv_units, seq_len, head_dim);
   const int units = static_cast<int>(kv_units * head_groups(group, hg));
   const bool forced = (flags & TQ_MATRIX_PRODUCTS) != 0;
+  const bool takes_mx = mx_shape(fmt, head_dim, group) && (flags & TQ_F32_PRODUCTS) == 0;
+  const int64_t blocks = std::max<int64_t>(1, (seq_len + mx::kStride - 1) / mx::kStride);
+  const int min_blocks = mx_min_blocks_per_split(head_dim);
+  const int ns4 = default_splits(units, seq_len, num_cus, 1);
   if (n_splits <= 0 && one_split(seq_len, fmt, head_dim)) {
-    if (!forced) return {SplitKernel::Fp32, 1, hg};
+    // the matrix kernel where its own plan is one split of enough blocks: 24
+    // layers x 8 KV heads x 512 4-bit tokens in groups of 4 at head_dim 128
+    // 7.3 us against 9.0, at 64 6.2 against 6.3, 2-bit rows 7.2 against 8.2
+    if (!forced && !(takes_mx && blocks / std::min<int64_t>(blocks, ns4) >= min_blocks)) return {SplitKernel::Fp32, 1, hg};
     n_splits = 1;
   }
-  if (mx_shape(fmt, head_dim, group) && (flags & TQ_F32_PRODUCTS) == 0) {
-    const int64_t blocks = std::max<int64_t>(1, (seq_len + mx::kStride - 1) / mx::kStride);
-    const int min_blocks = mx_min_blocks_per_split(head_dim);
-    const int ns4 = default_splits(units, seq_len, num_cus, 1);
+  if (takes_mx) {
     const int ns = n_splits > 0 ? n_splits : ns4;
     const bool runs = forced || blocks / std::min<int64_t>(blocks, ns) >= min_blocks;
     // Units of 8 heads where units of 4 would run: one read of the rows and
