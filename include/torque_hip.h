@@ -60,7 +60,16 @@ enum { TQ_ROTATE_KEYS = 1, TQ_ROTATE_VALUES = 2 };
  * merge sums the splits in a fixed order, so a decode returns bit-identical
  * outputs on every call, on any stream and in every graph replay, as the
  * reference's decode does (cache.py:98-140, mlx_ops.py:571-595). */
-enum { TQ_ROTATE_QUERY = 1, TQ_INVERSE_OUTPUT = 2, TQ_F32_PRODUCTS = 4, TQ_MATRIX_PRODUCTS = 8 };
+enum {
+  TQ_ROTATE_QUERY = 1,
+  TQ_INVERSE_OUTPUT = 2,
+  TQ_F32_PRODUCTS = 4,
+  TQ_MATRIX_PRODUCTS = 8,
+  /* default plan (n_splits <= 0): one split, so one launch, for packed
+   * sequences of at most 512 tokens and 8 iterations, for callers whose host
+   * pays more for the merge launch than the splits save the GPU */
+  TQ_ONE_LAUNCH = 16
+};
 
 int tq_abi_version(void);
 const char* tq_last_error(void);

@@ -37,9 +37,16 @@ def test_default_workspace_covers_every_plan():
     (24, 4, 4, 256, 3, 8192, 5),  # one round, 480 workgroups: more splits would save less than 1/16
     (1, 8, 4, 128, 3, 32768, 64),  # one round fills the CUs evenly: unchanged
     (24, 8, 1, 128, 4, 200, 1),  # short: one launch
-    (1, 8, 1, 128, 4, 512, 1),
+    (1, 8, 1, 128, 4, 384, 1),  # one split as far as it is the faster one on the GPU: 6 iterations
+    (1, 8, 1, 128, 4, 385, 4),
+    (1, 8, 4, 128, 3, 320, 1),  # 5 for units of several heads
+    (1, 8, 4, 128, 3, 321, 3),
     (1, 8, 1, 128, 4, 513, 5),
-    (1, 4, 4, 256, 4, 256, 1),
+    (1, 8, 1, 256, 4, 256, 1),  # 8 shorter ones
+    (1, 4, 4, 256, 4, 224, 1),
+    (1, 4, 4, 256, 4, 225, 2),
+    (24, 8, 4, 128, 3, 512, 1),  # more units than half of the CUs
+    (24, 8, 4, 128, 3, 513, 2),
     (1, 4, 4, 256, 4, 257, 3),
     (1, 4, 4, 64, 3, 512, 1),
     (1, 4, 4, 64, 3, 513, 5),
@@ -47,6 +54,18 @@ def test_default_workspace_covers_every_plan():
 ])
 def test_workgroups_spread_over_the_cus(layers, kv, group, dim, bits, seq, most):
     assert _splits(layers, kv, group, dim, bits, 0, seq) == most
+
+
+@pytest.mark.parametrize("dim,bits,most", [(64, 4, 512), (128, 2, 512), (128, 3, 512), (256, 4, 256)])
+@pytest.mark.parametrize("kv,group", [(8, 1), (4, 4), (4, 6)])
+def test_one_launch_on_request(dim, bits, most, kv, group):
+    """TQ_ONE_LAUNCH: one split up to 512 tokens and 8 iterations, on the kernel the call runs on without it."""
+    one = _lib.TQ_ONE_LAUNCH
+    assert _splits(1, kv, group, dim, bits, one, most) == 1 < _splits(1, kv, group, dim, bits, one, most + 1)
+    for seq in (100, most, most + 1, 20000):
+        name = lambda flags: _lib.split_kernel(kv, kv * group, dim, bits, flags, _lib.TQ_F16, seq, num_cus=CUS).split("<")[0]
+        assert name(one) == name(0)
+        assert _splits(1, kv, group, dim, bits, one, seq) == 1 or _splits(1, kv, group, dim, bits, 0, seq) == _splits(1, kv, group, dim, bits, one, seq)
 
 
 @pytest.mark.parametrize("layers,kv,group,dim,bits,seq,default", [

@@ -1805,20 +1805,28 @@ bool mx_shape(int fmt, int head_dim, int group) {
 // workgroup, writing its 128 KB of tables costs more than its loop saves.
 int mx_min_blocks_per_split(int head_dim) { return head_dim == 256 ? 8 : 4; }
 
-// Short packed sequences take one split by default: the workgroup of a head
-// group reads them in 8 iterations at most and finishes its rows itself, so
-// the call is one launch.  Measured on MI355X (one decode on the GPU, then
-// with its Python call): 256 tokens x 8 heads at head_dim 128 6.0 / 8.5 us
-// against 7.4 / 11.4 in 2 splits, 512 tokens 7.8 / 8.6 against 7.3 / 11.6, 768
-// tokens 9.9 / 9.9 against 7.5 / 11.5; at head_dim 256 256 tokens 8.9 / 9.0
-// against 9.2 / 11.3, 384 tokens 11.2 / 11.2 against 9.3 / 11.4; at head_dim
-// 64 512 tokens 6.5 / 8.6 against 7.3 / 11.2.
-constexpr int kShortBlocks = 8;
+// Short packed sequences take one split: the workgroup of a head group reads
+// them in few iterations and finishes its rows itself, so the call is one
+// launch.  The line is where that is as fast on the GPU.  Measured on MI355X
+// (graphs of decodes), one split against the splits of 128 tokens: at head_dim
+// 64 every case up to 512 tokens (4 iterations; 8 heads 5.3 us against 6.4);
+// at 128, groups of 1, 384 tokens (6) 6.6 against 7.1 but 448 7.2 against 7.1,
+// larger units 320 tokens (5) 7.5 against 7.7 but 384 3-bit tokens 8.1 against
+// 7.75; at 256, groups of 1, 256 tokens (8) 7.9 against 8.3, larger units 192
+// tokens (6) 8.0 against 8.5 but 256 9.2 against 9.0.  With more units than
+// half of the CUs the splits do not run side by side and one is faster up to
+// 512 tokens (24 layers x 8 heads, 512 3-bit tokens at 128 9.6 against 15.5).
+// A caller whose host pays for the second launch asks for TQ_ONE_LAUNCH: 512
+// tokens x 8 heads at head_dim 128 take 7.6 us on the GPU in one split and 7.1
+// in 4, and 8.6 against 11.6 with the Python call around them.
 constexpr int kShortTokens = 512;
+constexpr int kShortIterations = 8;
 
-bool one_split(int64_t seq_len, int fmt, int head_dim) {
-  const bool packed = fmt == 2 || fmt == 3 || fmt == 4;
-  return packed && seq_len <= std::min(kShortTokens, kShortBlocks * decode_block_rows(fmt, head_dim));
+bool one_split(int64_t seq_len, int fmt, int head_dim, int hg, int64_t units, int num_cus, bool one_launch) {
+  if (fmt != 2 && fmt != 3 && fmt != 4) return false;
+  int iterations = kShortIterations;
+  if (!one_launch && 2 * units <= num_cus) iterations = (head_dim == 256 ? 8 : 6) - (hg > 1);
+  return seq_len <= std::min(kShortTokens, iterations * decode_block_rows(fmt, head_dim));
 }
 
 // Split kernel, split count and heads per unit of a decode over kv_units
@@ -1839,7 +1847,8 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
   const int64_t blocks = std::max<int64_t>(1, (seq_len + mx::kStride - 1) / mx::kStride);
   const int min_blocks = mx_min_blocks_per_split(head_dim);
   const int ns4 = default_splits(units, seq_len, num_cus, 1);
-  if (n_splits <= 0 && one_split(seq_len, fmt, head_dim)) {
+  const bool one_launch = forced || (flags & TQ_ONE_LAUNCH) != 0;
+  if (n_splits <= 0 && one_split(seq_len, fmt, head_dim, hg, units, num_cus, one_launch)) {
     // the matrix kernel where its own plan is one split of enough blocks: 24
     // layers x 8 KV heads x 512 4-bit tokens in groups of 4 at head_dim 128
     // 7.3 us against 9.0, at 64 6.2 against 6.3, 2-bit rows 7.2 against 8.2

@@ -36,6 +36,7 @@ TQ_ROTATE_QUERY = 1
 TQ_INVERSE_OUTPUT = 2
 TQ_F32_PRODUCTS = 4
 TQ_MATRIX_PRODUCTS = 8
+TQ_ONE_LAUNCH = 16
 
 _p = ctypes.c_void_p
 _i = ctypes.c_int

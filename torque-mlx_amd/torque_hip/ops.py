@@ -82,7 +82,8 @@ def plan_splits(
     bit_width: int = 0,
     flags: int = 0,
 ) -> int:
-    """The library's default split count for a decode over ``bit_width``-bit rows (0: dense rows)."""
+    """The library's default split count for a decode over ``bit_width``-bit rows (0: dense rows): the fastest on the
+    GPU, which a captured decode passes as ``n_splits``."""
     return _lib.call(
         "tq_decode_default_splits", num_layers, kv_heads, query_heads, head_dim, bit_width, flags, seq_len, num_cus(dev)
     )
@@ -134,12 +135,16 @@ def packed_decode(
     take it (the library adds the flag), so their split plan does too.
     ``matrix_products`` (TQ_MATRIX_PRODUCTS) runs the matrix kernel wherever it
     can, also where the default plan leaves too few rows per split for it.
+    Without ``n_splits`` a short sequence takes one split and one launch
+    (TQ_ONE_LAUNCH), eager and captured alike; ``plan_splits`` gives the count
+    that is fastest on the GPU alone.
     """
     dev = query.device
     scaled = key_scales is not None or value_scales is not None
     flags = (_lib.TQ_ROTATE_QUERY if rotate_query else 0) | (_lib.TQ_INVERSE_OUTPUT if inverse_output else 0)
     flags |= _lib.TQ_F32_PRODUCTS if f32_products or scaled else 0
     flags |= _lib.TQ_MATRIX_PRODUCTS if matrix_products else 0
+    flags |= _lib.TQ_ONE_LAUNCH  # this call costs the host more than the splits of a short sequence save
     n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
     ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
     if out is None:
@@ -214,6 +219,7 @@ def packed_decode_append(
     append_flags = (_lib.TQ_ROTATE_KEYS if rotate_keys else 0) | (_lib.TQ_ROTATE_VALUES if rotate_values else 0)
     decode_flags = (_lib.TQ_ROTATE_QUERY if rotate_query else 0) | (_lib.TQ_INVERSE_OUTPUT if inverse_output else 0)
     decode_flags |= _lib.TQ_MATRIX_PRODUCTS if matrix_products else 0
+    decode_flags |= _lib.TQ_ONE_LAUNCH  # as in packed_decode
     n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
     ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
     if out is None:
