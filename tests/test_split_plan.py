@@ -94,3 +94,11 @@ def test_one_split_of_many_units_keeps_the_matrix_kernel(layers, kv, group, dim,
         assert "mx" in name(seq, layers)
         assert "mx" not in name(seq, 1)
     assert "mx" not in name(384, layers)
+
+
+@pytest.mark.parametrize("kv,group,dim,bits,seq", [(4, 7, 64, 3, 30000), (8, 3, 128, 4, 32768), (2, 5, 256, 2, 20000)])
+def test_explicit_counts_of_few_workgroups_keep_units_of_one(kv, group, dim, bits, seq):
+    """An odd group is cut into units of 4 heads only where its units of 1 would be more workgroups than CUs."""
+    heads = lambda n: _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, n_splits=n, num_cus=CUS).rstrip(">").split(",")[2]
+    most = CUS // (kv * group)
+    assert [heads(n) for n in (1, most, most + 1, 64, 0)] == ["1", "1", "4", "4", "4"]
