@@ -1,9 +1,9 @@
 """Row kernels on calls larger than one launch.
 
-The rotation, append (rotate, quantize, pack) and unpack entry points cut a
-call into launches of at most 2^20 workgroups (a HIP launch holds at most
-2^32 - 1 work-items): at whole (layer, head) groups, or at token ranges when
-one group alone is larger.  Each case here crosses that size and is checked
+The rotation and unpack entry points cut a call into launches of at most 2^20
+workgroups, the append (rotate, quantize, pack) entry points into launches of at
+most 2^23 rows of a stream (a HIP launch holds at most 2^32 - 1 work-items): at
+whole (layer, head) groups, or at token ranges when one group alone is larger.  Each case here crosses that size and is checked
 bit-exact against the same work done by several smaller calls that each fit
 one launch (cut at other points), and against the CPU oracle on the rows
 around every cut.
@@ -23,6 +23,7 @@ pytestmark = pytest.mark.gpu
 
 MAX_BLOCKS = 1 << 20  # workgroups per launch of the row kernels
 WAVES = 4  # wavefronts per workgroup
+MAX_APPEND_ROWS = 1 << 23  # rows of a stream per launch of the append kernels
 D = 64
 
 
@@ -84,8 +85,8 @@ def _oracle_words(x_rows: np.ndarray, sl, sr, bnd: np.ndarray, bits: int) -> np.
 @pytest.mark.parametrize(
     ("kv_heads", "seq_new"),
     [
-        (1, MAX_BLOCKS * WAVES // 2 + 37),  # one group larger than a launch: cut at tokens
-        (5, 1_000_000),  # two groups per launch: cut at groups
+        (1, MAX_APPEND_ROWS + 37),  # one group larger than a launch: cut at tokens
+        (5, 4_000_000),  # two groups per launch: cut at groups
     ],
 )
 def test_append_past_one_launch(hip_device, kv_heads, seq_new):
@@ -112,8 +113,7 @@ def test_append_past_one_launch(hip_device, kv_heads, seq_new):
     torch.cuda.synchronize()
     assert torch.equal(kc, kp) and torch.equal(vc, vp)
     assert not kc[:, :offset].any() and not kc[:, offset + seq_new :].any()
-    max_rows = MAX_BLOCKS * WAVES // 2
-    cuts = [max_rows, cut] if kv_heads == 1 else [cut]
+    cuts = [MAX_APPEND_ROWS, cut] if kv_heads == 1 else [cut]
     idx = _near(cuts, seq_new)
     for h in {0, kv_heads - 1}:
         for src, dst in ((keys, kc), (values, vc)):
