@@ -154,7 +154,8 @@ int tq_decode_default_splits(int num_layers, int kv_heads, int query_heads, int 
  * decode `flags`, a query of `query_dtype`, seq_len tokens and n_splits
  * (<= 0: the default) launches on num_cus compute units (<= 0: the current
  * device's): "decode_mx_kernel<D,QF16>" (the float16-split matrix kernel;
- * "decode_mx_kernel<D,QF16,2>" for 2-bit rows) or
+ * "decode_mx_kernel<D,QF16,2>" for 2-bit rows, "decode_mx_kernel<D,QF16,bits,8>"
+ * for units of 8 query heads) or
  * "decode_kernel<PackedB<bits>,D,<heads per group>>" (the float32 kernel;
  * tq_decode_scaled always runs this one).  For profiles and benchmarks; no
  * reference counterpart.  NULL on bad arguments (tq_last_error). */

@@ -102,3 +102,14 @@ def test_explicit_counts_of_few_workgroups_keep_units_of_one(kv, group, dim, bit
     heads = lambda n: _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, n_splits=n, num_cus=CUS).rstrip(">").split(",")[2]
     most = CUS // (kv * group)
     assert [heads(n) for n in (1, most, most + 1, 64, 0)] == ["1", "1", "4", "4", "4"]
+
+
+@pytest.mark.parametrize("kv,group,dim,bits,seq", [(4, 8, 128, 4, 30001), (8, 16, 128, 2, 32768), (2, 24, 256, 4, 131072), (8, 8, 64, 4, 32768)])
+def test_units_of_8_have_their_own_name(kv, group, dim, bits, seq):
+    """The 8-head instance is named apart from the 4-head one, so an explicit count shows which of them it runs."""
+    name = lambda n, g=group: _lib.split_kernel(kv, kv * g, dim, bits, 0, _lib.TQ_F16, seq, n_splits=n, num_cus=CUS)
+    eight = f"decode_mx_kernel<{dim},true,{bits},8>"
+    default = _splits(1, kv, group, dim, bits, 0, seq)
+    assert name(0) == name(default) == eight
+    assert name(1) == f"decode_mx_kernel<{dim},true{'' if bits == 4 else ',2'}>"  # too few workgroups for units of 8
+    assert name(1, 4) == name(1)

@@ -2769,7 +2769,7 @@ const char* tq_decode_split_kernel(int num_layers, int kv_heads, int query_heads
   const KernelChoice kc = choose_kernel(kv_units, seq_len, n_splits, bits, head_dim, group, flags, num_cus);
   if (kc.kernel == SplitKernel::Mx)
     name = "decode_mx_kernel<" + std::to_string(head_dim) + "," + (query_dtype == TQ_F16 ? "true" : "false") +
-           (bits == 4 ? ">" : "," + std::to_string(bits) + ">");
+           (kc.hg == 8 ? "," + std::to_string(bits) + ",8>" : bits == 4 ? ">" : "," + std::to_string(bits) + ">");
   else if (fp32_tokens_per_iter(bits, head_dim, kc.hg, seq_len, kc.n_splits) == kWideTokensPerIter)
     name = "decode_kernel<PackedB4,256,4," + std::to_string(kWideTokensPerIter) + ">";
   else
