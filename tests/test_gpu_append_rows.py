@@ -5,6 +5,10 @@ at head_dim 64, 128, 256) and groups that end inside a wavefront,
 sources that are not 16-byte aligned, quotients that tie with a boundary, values without an ordinary quotient (zeros,
 subnormals, infinities, NaN), and codebooks that the bucket lookup cannot take (equal, unordered, infinite boundaries).
 Whole-number outputs: no tolerance.
+
+The forms with per-vector scales and those that write centroid values run here above the line, where the other tests of
+those entry points stay below it: bit for bit the same as calls of few rows, codes and centroids against the oracle on
+the kernel's own scales.
 """
 
 from __future__ import annotations
@@ -129,3 +133,112 @@ def test_signs_of_any_size(hip_device, head_dim):
     signs = [(s * rng.uniform(0.5, 2.0, size=head_dim)).astype(np.float32) for s in o.rotation_signs_from_seed(head_dim, 4)]
     bnd = o.codebook_boundaries(o.build_gaussian_codebook(4, sample_size=5000, seed=1))
     _check(x, signs, bnd, 4, seq_new=2100)
+
+
+def _stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def _codebooks(bits):
+    books = [o.build_gaussian_codebook(bits, sample_size=5000, seed=s) for s in (1, 2)]
+    return [torch.from_numpy(np.asarray(a, dtype=np.float32)).cuda() for b in books for a in (o.codebook_boundaries(b), b)]
+
+
+def _sources(rows, head_dim, dtype, shift, seed):
+    """Two streams of rows over a few decades of norms, `shift` elements off a 16-byte boundary, with rows whose mean
+    square is zero, infinite, subnormal or no number."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    out = []
+    for _ in range(2):
+        x = torch.randn(rows, head_dim, generator=g, device="cuda") * torch.randn(rows, 1, generator=g, device="cuda").exp()
+        x[7], x[rows - 2], x[100, 3], x[4096 % rows, 5], x[9] = 0.0, 0.0, float("inf"), float("nan"), x[9] * 1e-23
+        buf = torch.zeros(rows * head_dim + shift, dtype=dtype, device="cuda")
+        buf[shift:] = x.reshape(-1).to(dtype)
+        out.append(buf[shift:].view(rows, head_dim))
+    return out
+
+
+def _type(x):
+    import torque_hip as th
+
+    return th._lib.TQ_F16 if x.dtype == torch.float16 else th._lib.TQ_F32
+
+
+FORMS = [(2053, torch.float16, 0, 3), (2053, torch.float32, 1, 3), (4500, torch.float32, 0, 3), (4500, torch.float16, 3, 0), (9001, torch.float16, 0, 1)]
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("head_dim", DIMS)
+@pytest.mark.parametrize("rows,dtype,shift,flags", FORMS)
+def test_scaled_rows(hip_device, bits, head_dim, rows, dtype, shift, flags):
+    import torque_hip as th
+
+    keys, values = _sources(rows, head_dim, dtype, shift, bits + head_dim)
+    signs = o.rotation_signs_from_seed(head_dim, 6)
+    left, right = (torch.from_numpy(s).cuda() for s in signs)
+    kb, _, vb, _ = _codebooks(bits)
+    words = head_dim * bits // 32
+
+    def append(cuts):
+        codes = [torch.full((rows + 2, words), -1, dtype=torch.int32, device="cuda") for _ in range(2)]
+        scales = [torch.full((rows + 2,), -1.0, device="cuda") for _ in range(2)]
+        for t0, t1 in cuts:
+            th._lib.call("tq_append_scaled", keys[t0:t1].data_ptr(), values[t0:t1].data_ptr(), _type(keys), 1, 1, t1 - t0, head_dim, bits,
+                         left.data_ptr(), right.data_ptr(), flags, kb.data_ptr(), vb.data_ptr(), codes[0].data_ptr(), codes[1].data_ptr(),
+                         scales[0].data_ptr(), scales[1].data_ptr(), rows + 2, 1 + t0, _stream())
+        return codes, scales
+
+    codes, scales = append([(0, rows)])
+    few_codes, few_scales = append([(t, min(t + 1000, rows)) for t in range(0, rows, 1000)])
+    for i, (x, rotate, bnd) in enumerate(((keys, flags & 1, kb), (values, flags & 2, vb))):
+        assert torch.equal(codes[i], few_codes[i]) and torch.equal(scales[i].view(torch.int32), few_scales[i].view(torch.int32))
+        assert codes[i][0].eq(-1).all() and codes[i][-1].eq(-1).all() and scales[i][0] == scales[i][-1] == -1.0
+        with np.errstate(all="ignore"):
+            y = x.float().cpu().numpy()
+            y = o.rotation_apply(y, *signs) if rotate else y
+            s = scales[i][1:-1].cpu().numpy()
+            exp, _ = o.quantize_scaled(y, bnd.cpu().numpy(), s)
+        np.testing.assert_array_equal(codes[i][1:-1].cpu().numpy().view(np.uint32), o.pack_indices_batched(exp, bits))
+        ordinary = np.isfinite(y).all(axis=1) & (np.abs(y).max(axis=1) > 1e-15)  # whose squares float32 holds
+        np.testing.assert_allclose(s[ordinary], o.rms_scales(y[ordinary]), rtol=3e-6)  # as test_gpu_scaled.py
+        assert s[7] == s[rows - 2] == 1.0 and ordinary.sum() >= rows - 6
+
+
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("head_dim", DIMS)
+@pytest.mark.parametrize("rows,dtype,shift,flags", FORMS)
+def test_dequantized_rows(hip_device, bits, head_dim, rows, dtype, shift, flags, scaled):
+    import torque_hip as th
+
+    keys, values = _sources(rows, head_dim, dtype, shift, bits + head_dim)
+    left, right = (torch.from_numpy(s).cuda() for s in o.rotation_signs_from_seed(head_dim, 6))
+    kb, kc, vb, vc = _codebooks(bits)
+    words = head_dim * bits // 32
+    name = "_scaled" if scaled else ""
+
+    def dequantize(cuts, off=0):
+        out = [torch.full((rows * head_dim + 8,), 99.0, device="cuda") for _ in range(2)]
+        for t0, t1 in cuts:
+            ptrs = [x[off + t0 * head_dim :].data_ptr() for x in out]
+            th._lib.call("tq_quantize_dequantize" + name, keys[t0:t1].data_ptr(), values[t0:t1].data_ptr(), _type(keys), t1 - t0, head_dim,
+                         bits, left.data_ptr(), right.data_ptr(), flags, kb.data_ptr(), vb.data_ptr(), kc.data_ptr(), vc.data_ptr(), *ptrs,
+                         _stream())
+        for x in out:
+            assert x[:off].eq(99.0).all() and x[off + rows * head_dim :].eq(99.0).all()
+        return [x[off : off + rows * head_dim].view(rows, head_dim) for x in out]
+
+    got = dequantize([(0, rows)])
+    few = dequantize([(t, min(t + 1000, rows)) for t in range(0, rows, 1000)])
+    moved = dequantize([(0, rows)], off=1)  # outputs off a 16-byte boundary
+    # the packing form's codes (and scales), which the tests above compare with the oracle
+    codes = [torch.zeros(rows, words, dtype=torch.int32, device="cuda") for _ in range(2)]
+    scales = [torch.zeros(rows, device="cuda") for _ in range(2)]
+    extra = [s.data_ptr() for s in scales] if scaled else []
+    th._lib.call("tq_append" + name, keys.data_ptr(), values.data_ptr(), _type(keys), 1, 1, rows, head_dim, bits, left.data_ptr(),
+                 right.data_ptr(), flags, kb.data_ptr(), vb.data_ptr(), codes[0].data_ptr(), codes[1].data_ptr(), *extra, rows, 0, _stream())
+    for i, cent in enumerate((kc, vc)):
+        index = torch.from_numpy(o.unpack_indices_batched(codes[i].cpu().numpy().view(np.uint32), bits, head_dim).astype(np.int64)).cuda()
+        want = cent[index] * scales[i][:, None] if scaled else cent[index]
+        for y in (got[i], few[i], moved[i]):
+            assert torch.equal(y.view(torch.int32), want.view(torch.int32))
