@@ -114,3 +114,37 @@ def test_captured_noalloc_replays(hip_device):
         np.testing.assert_array_equal(got, ref, err_msg=f"replay {rep}")
         _noalloc(other, q_other, out_other)
         torch.cuda.synchronize(hip_device)
+
+
+def test_capture_after_an_explicit_count(hip_device):
+    """A default-plan decode is captured on a stream whose workspace an explicit count of as many splits left there: a
+    capture cannot grow it to what the default plan needs at any length, and has no need to."""
+    from torque_hip import ops
+
+    cache = _cache(hip_device, 3, 128, 8, 4000, seed=24)
+    st = cache._store
+    q = torch.randn((1, 8, 128), generator=torch.Generator(device=hip_device).manual_seed(7), device=hip_device)
+
+    def decode(n_splits):
+        return ops.packed_decode(q, num_layers=1, query_heads=8, kv_heads=8, head_dim=128, bit_width=3, key_codes=st.key_codes,
+                                 value_codes=st.value_codes, capacity=st.capacity, seq_len=st.length,
+                                 key_centroids=st.key_centroids, value_centroids=st.value_centroids, signs_left=st.signs_left,
+                                 signs_right=st.signs_right, rotate_query=True, inverse_output=True, n_splits=n_splits)
+
+    expected = decode(None)
+    n_splits = ops.plan_splits(1, 8, 8, 128, st.length, hip_device, bit_width=3)
+    assert ops._workspace_bytes(1, 8, 8, 128, n_splits, ops.num_cus(hip_device)) < ops._workspace_bytes(1, 8, 8, 128, 0, ops.num_cus(hip_device))
+    side = torch.cuda.Stream(hip_device)
+    with torch.cuda.stream(side):
+        ops.Workspace._pool.pop((hip_device, side.cuda_stream), None)  # an earlier stream's of the same handle
+        decode(n_splits)
+    torch.cuda.synchronize(hip_device)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = decode(None)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize(hip_device)
+        assert torch.equal(out, expected)
+        decode(2)

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 from functools import lru_cache
 from math import sqrt
-from typing import Any
+from typing import Any, Callable
 
 import torch
 
@@ -55,11 +55,14 @@ class Workspace:
     _pool: dict[tuple[torch.device, int], torch.Tensor] = {}
 
     @classmethod
-    def get(cls, nbytes: int, dev: torch.device) -> torch.Tensor:
+    def get(cls, nbytes: int, dev: torch.device, least: Callable[[], int] | None = None) -> torch.Tensor:
+        """At least ``nbytes``; a stream capture, which cannot grow it, makes do with ``least()`` bytes."""
         key = (dev, stream_handle(dev))
         buf = cls._pool.get(key)
         if buf is None or buf.numel() < nbytes:
             if buf is not None:
+                if least is not None and torch.cuda.is_current_stream_capturing() and buf.numel() >= least():
+                    return buf
                 torch.cuda.current_stream(dev).synchronize()
             buf = torch.zeros(max(nbytes, 1 << 16), dtype=torch.uint8, device=dev)
             cls._pool[key] = buf
@@ -94,9 +97,27 @@ def _workspace_bytes(num_layers: int, kv_heads: int, query_heads: int, head_dim:
     return int(_lib.call("tq_decode_workspace_bytes", num_layers, kv_heads, query_heads, head_dim, n_splits, cus))
 
 
-def workspace_for(num_layers: int, kv_heads: int, query_heads: int, head_dim: int, n_splits: int, dev: torch.device) -> torch.Tensor:
-    """A workspace of ``n_splits`` splits (0: of the default plan at any length)."""
-    return Workspace.get(_workspace_bytes(num_layers, kv_heads, query_heads, head_dim, n_splits, num_cus(dev)), dev)
+def workspace_for(
+    num_layers: int,
+    kv_heads: int,
+    query_heads: int,
+    head_dim: int,
+    n_splits: int,
+    dev: torch.device,
+    seq_len: int | None = None,
+    *,
+    bit_width: int = 0,
+    flags: int = 0,
+) -> torch.Tensor:
+    """A workspace of ``n_splits`` splits (0: of the default plan at any length, or in a stream capture, where the
+    stream's workspace holds no more, at ``seq_len``)."""
+    shape = (num_layers, kv_heads, query_heads, head_dim)
+    cus = num_cus(dev)
+
+    def least() -> int:
+        return _workspace_bytes(*shape, plan_splits(*shape, seq_len, dev, bit_width=bit_width, flags=flags), cus)
+
+    return Workspace.get(_workspace_bytes(*shape, n_splits, cus), dev, None if n_splits > 0 or seq_len is None else least)
 
 
 def packed_decode(
@@ -146,7 +167,7 @@ def packed_decode(
     flags |= _lib.TQ_MATRIX_PRODUCTS if matrix_products else 0
     flags |= _lib.TQ_ONE_LAUNCH  # this call costs the host more than the splits of a short sequence save
     n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
-    ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
+    ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev, seq_len, bit_width=bit_width, flags=flags)
     if out is None:
         out = torch.empty((num_layers, query_heads, head_dim), dtype=torch.float32, device=dev)
     if scaled and (key_scales is None or value_scales is None):
@@ -221,7 +242,8 @@ def packed_decode_append(
     decode_flags |= _lib.TQ_MATRIX_PRODUCTS if matrix_products else 0
     decode_flags |= _lib.TQ_ONE_LAUNCH  # as in packed_decode
     n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
-    ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
+    ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev, seq_len, bit_width=bit_width,
+                       flags=decode_flags)
     if out is None:
         out = torch.empty((num_layers, query_heads, head_dim), dtype=torch.float32, device=dev)
     _lib.call(
@@ -278,7 +300,7 @@ def dense_decode(
     """One ``tq_decode_dense`` launch: dense fp16/fp32 K/V slabs [L, Hkv, capacity, D]."""
     dev = query.device
     n_splits = max(n_splits or 0, 0)  # 0: the library's default plan
-    ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev)
+    ws = workspace_for(num_layers, kv_heads, query_heads, head_dim, n_splits, dev, seq_len)
     if out is None:
         out = torch.empty((num_layers, query_heads, head_dim), dtype=torch.float32, device=dev)
     flags = (_lib.TQ_ROTATE_QUERY if rotate_query else 0) | (_lib.TQ_INVERSE_OUTPUT if inverse_output else 0)
