@@ -50,9 +50,12 @@ enum { TQ_ROTATE_KEYS = 1, TQ_ROTATE_VALUES = 2 };
  * The split kernel (no reference counterpart): the float16-split matrix
  * kernel can run for groups of 4, 8, 12, ... query heads with 4-bit rows at
  * head_dim 64 / 128 / 256 or 2-bit rows at head_dim 128, and by default does
- * where its split plan gives every split at least 4 blocks of 128 rows (8 at
- * head_dim 256); elsewhere the float32 split kernel runs.  Both accumulate in float32.  TQ_F32_PRODUCTS selects
- * the float32 kernel, TQ_MATRIX_PRODUCTS the matrix kernel wherever it can
+ * where its split plan in units of 4 heads gives every split at least 4 blocks
+ * of 128 rows (8 at head_dim 256); elsewhere the float32 split kernel runs.
+ * Groups that are a multiple of 8 then run in units of 8 heads, half as many
+ * units in up to twice as many splits, each of which may have half as many
+ * blocks.  Both kernels accumulate in float32.  TQ_F32_PRODUCTS selects the
+ * float32 kernel, TQ_MATRIX_PRODUCTS the matrix kernel wherever it can
  * run (the two exclude each other: TQ_ERR_BAD_ARG).  tq_decode_scaled always
  * runs the float32 split kernel.
  *
@@ -142,11 +145,13 @@ int tq_unpack_dequantize_scaled(const uint32_t* codes, const float* scales, int6
                                 hipStream_t stream);
 
 /* Split count a decode call over `bits`-bit rows (0 for dense rows) with
- * decode `flags` (passed explicitly it runs the same split kernel, short
- * sequences of one split aside) uses when n_splits <= 0 is passed, on num_cus compute units
- * (<= 0: the current device's).  The sequence is dealt out to the splits in
- * blocks of one workgroup iteration (split s takes blocks s, s + n, s + 2n,
- * ...); an explicit n_splits above the number of blocks is lowered to it. */
+ * decode `flags` uses when n_splits <= 0 is passed, on num_cus compute units
+ * (<= 0: the current device's).  Passed explicitly, this count runs the same
+ * split kernel, except that a short sequence's count of 1 may run the matrix
+ * kernel where the default runs the float32 kernel.  The sequence is dealt out
+ * to the splits in blocks of one workgroup iteration (split s takes blocks s,
+ * s + n, s + 2n, ...); an explicit n_splits above the number of blocks is
+ * lowered to it. */
 int tq_decode_default_splits(int num_layers, int kv_heads, int query_heads, int head_dim, int bits, int flags,
                              int64_t seq_len, int num_cus);
 

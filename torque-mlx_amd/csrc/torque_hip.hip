@@ -105,7 +105,8 @@ __global__ __launch_bounds__(kBlock) void fwht_kernel(const T* __restrict__ x, f
 
 
 // Division of a 32-bit row number by the tokens per group, as a multiply-high
-// and a shift with constants from the host (d >= 1, n < 2^31).
+// and a shift with constants from the host (d >= 1, n < 2^31): Granlund and
+// Montgomery's division by invariant integers.
 struct FastDiv {
   uint32_t mul, shift, d;
   __device__ uint32_t quot(uint32_t n) const { return (__umulhi(n, mul) + n) >> shift; }
@@ -1636,10 +1637,10 @@ constexpr int kMergeWork = 12;  // the merge launch that more than one split add
 // what counts is the work of the CU with the most.  Starting from the
 // one-round count ns0, take the count that makes it smallest, if that is at
 // least 1/16 less.  Measured on MI355X, 24 layers x 8 KV heads: 3-bit rows at
-// head_dim 128 x 8192 tokens, groups of 4, 75 us at 2 splits, 59 at 4 (768
-// workgroups, 3 to a CU), 64 at 5, 63 at 8; 4-bit rows, groups of 1, 60, 47,
-// 50, 47; at head_dim 64, groups of 2, 38, 31, 33, 31.  Over 20 random shapes
-// whose count it changes: 1.08 to 1.66 times as fast.  The overheads keep it
+// head_dim 128 x 8192 tokens, groups of 4, 74 us at 2 splits, 60 at 4 (768
+// workgroups, 3 to a CU), 64 at 5, 63 at 8; 4-bit rows, groups of 1, 57, 45,
+// 47, 44; at head_dim 64, groups of 2, 36, 30, 31, 31.  Over 24 random shapes
+// whose count it changes: 1.03 to 1.41 times as fast.  The overheads keep it
 // from short sequences, where more splits lose (640 units x 2235 tokens at
 // head_dim 256: 65 us at 1 split, 67.5 at 2).
 int balanced_splits(int units, int ns0, int64_t blocks, int num_cus) {
@@ -1789,15 +1790,15 @@ int fp32_tokens_per_iter(int fmt, int head_dim, int hg, int64_t seq_len, int64_t
   return 8 * iters(kWideTokensPerIter) < 5 * iters(kTokensPerIter) ? kWideTokensPerIter : kTokensPerIter;
 }
 
-// Shapes the matrix-core split kernel takes: groups of 4 query heads with
-// 4-bit rows at head_dim 64 / 128 / 256 or 2-bit rows at head_dim 128.
+// Shapes the matrix-core split kernel takes: groups of a multiple of 4 query
+// heads with 4-bit rows at head_dim 64 / 128 / 256 or 2-bit rows at head_dim 128.
 bool mx_shape(int fmt, int head_dim, int group) {
   return group % 4 == 0 && ((fmt == 4 && (head_dim == 64 || head_dim == 128 || head_dim == 256)) ||
-                     (fmt == 2 && head_dim == 128));
+                            (fmt == 2 && head_dim == 128));
 }
 
-// Fewest 128-row blocks per split at which the matrix-core kernel runs by
-// default.  Measured on MI355X (wall time per decode, each kernel on its own
+// Fewest 128-row blocks per split, in units of 4 heads, at which the
+// matrix-core kernel runs by default.  Measured on MI355X (wall time per decode, each kernel on its own
 // default split plan): at head_dim 128 it is level with the float32 kernel at
 // 2 blocks per split and ahead from 4 (0.6 us at 16K tokens x 8 KV heads,
 // 1.6 us at 32K); at head_dim 256 it trails at 1-4 blocks (0.2-1.6 us) and
