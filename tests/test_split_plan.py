@@ -113,3 +113,16 @@ def test_units_of_8_have_their_own_name(kv, group, dim, bits, seq):
     assert name(0) == name(default) == eight
     assert name(1) == f"decode_mx_kernel<{dim},true{'' if bits == 4 else ',2'}>"  # too few workgroups for units of 8
     assert name(1, 4) == name(1)
+
+
+@pytest.mark.parametrize("layers,kv,group,dim,bits,seq,most", [
+    (16, 8, 8, 128, 4, 1309, 1), (16, 8, 8, 128, 4, 5376, 1), (16, 8, 8, 128, 4, 5377, 2),  # 128 units: from 43 blocks on
+    (24, 4, 8, 128, 2, 768, 1), (12, 8, 8, 64, 4, 3968, 1), (12, 8, 8, 128, 4, 8192, 2),  # 96 units: from 32
+    (9, 8, 8, 128, 4, 2176, 1), (9, 8, 8, 128, 4, 2177, 3),  # 72 units, 3 splits: from 18
+    (16, 8, 8, 256, 4, 3968, 1), (16, 8, 8, 256, 4, 3969, 2),  # head_dim 256: from 32
+    (8, 8, 8, 128, 4, 1024, 4),  # units of 4 have splits of their own to merge
+])
+def test_units_of_8_take_splits_that_pay_for_their_merge(layers, kv, group, dim, bits, seq, most):
+    assert _splits(layers, kv, group, dim, bits, 0, seq) == most
+    name = _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=layers, n_splits=0, num_cus=CUS)
+    assert name == f"decode_mx_kernel<{dim},true,{bits},8>"

@@ -1830,6 +1830,19 @@ bool one_split(int64_t seq_len, int fmt, int head_dim, int hg, int64_t units, in
   return seq_len <= std::min(kShortTokens, iterations * decode_block_rows(fmt, head_dim));
 }
 
+// Whether ns splits of units of 8 heads pay for the merge that they need where
+// units of 4 fill the CUs with one split each: the blocks they take off a
+// workgroup against partial results in proportion to the units.  Measured on
+// MI355X, units of 8 in one split / in ns (units of 4): 128 units, 4-bit rows
+// at head_dim 128, 1024 tokens 10.4 / 17.8 us (10.7), 4096 24.5 / 27.4 (29.7),
+// 6144 35.1 / 33.7 (41.2); 96 units 3072 18.4 / 20.4 (19.4), 4096 22.7 / 22.7
+// (24.1); 72 units, 3 splits 2048 13.8 / 15.6 (13.9), 3072 18.2 / 17.1 (18.8);
+// the same lines at head_dim 64 and for 2-bit rows; at 256, 128 units, 3072
+// tokens 39.0 / 42.0 (43.6), 4096 49.7 / 48.6 (54.1).
+bool splits_pay_units_of_8(int units, int ns, int64_t blocks, int head_dim) {
+  return blocks * (ns - 1) * (head_dim == 256 ? 8 : 6) >= static_cast<int64_t>(units) * ns;
+}
+
 // Split kernel, split count and heads per unit of a decode over kv_units
 // (layers x KV heads) with decode `flags` (n_splits <= 0: the default count
 // for the chosen kernel).
@@ -1875,7 +1888,8 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
     // -> 23.8, 24 layers x 2 x 8192 at 256 59.7 -> 33.4.  An explicit count
     // has to give more than half of the CUs a workgroup.
     if (group % 8 == 0) {
-      const int ns8 = default_splits(units / 2, seq_len, num_cus, 1);
+      int ns8 = default_splits(units / 2, seq_len, num_cus, 1);
+      if (ns4 == 1 && !splits_pay_units_of_8(units / 2, ns8, blocks, head_dim)) ns8 = 1;
       if (n_splits <= 0 || n_splits == ns8) {
         if (forced || blocks / std::min<int64_t>(blocks, ns4) >= min_blocks) return {SplitKernel::Mx, ns8, 8};
       } else if (forced || (runs && static_cast<int64_t>(units / 2) * n_splits > num_cus / 2)) {
