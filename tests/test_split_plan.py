@@ -126,3 +126,17 @@ def test_units_of_8_take_splits_that_pay_for_their_merge(layers, kv, group, dim,
     assert _splits(layers, kv, group, dim, bits, 0, seq) == most
     name = _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=layers, n_splits=0, num_cus=CUS)
     assert name == f"decode_mx_kernel<{dim},true,{bits},8>"
+
+
+@pytest.mark.parametrize("units,group,dim,bits,seq,most,cut", [
+    (96, 5, 128, 3, 768, 1, True), (96, 5, 128, 3, 1536, 1, True), (96, 5, 128, 3, 2048, 2, True),
+    (128, 3, 128, 3, 768, 1, True), (128, 3, 128, 3, 1024, 4, True), (64, 3, 128, 3, 768, 6, True),  # 64 units: CUs left idle
+    (96, 7, 64, 4, 768, 1, True), (128, 6, 256, 4, 768, 1, True), (128, 5, 128, 3, 600, 1, True),
+    (128, 4, 128, 3, 768, 4, True),  # units that divide the group keep their plan
+    (64, 7, 128, 0, 767, 1, False), (64, 7, 128, 0, 768, 4, True), (96, 5, 128, 0, 768, 1, True),  # dense rows: cut from 768 tokens on
+])
+def test_cut_groups_take_splits_that_pay_for_their_merge(units, group, dim, bits, seq, most, cut):
+    assert _splits(units, 1, group, dim, bits, 0, seq) == most
+    if bits:
+        name = _lib.split_kernel(1, group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=units, n_splits=0, num_cus=CUS)
+        assert name == f"decode_kernel<PackedB{bits},{dim},{4 if cut else 1}>"

@@ -1596,13 +1596,18 @@ __global__ __launch_bounds__(kStreamThreads) void stream_read_kernel(const uint4
 // -> 26.0; 16 x 8 heads at 64, 23236 tokens, groups of 3 124 -> 57; 10 M
 // elements saved 18.6 -> 16.1, but 4.2 M 9.3 -> 10.1 and 5.1 M (dense rows)
 // 7.5 -> 8.4.
+// Dense rows, which units of 1 and 2 read without table lookups, are cut from
+// 768 tokens on: 64 units x 7 heads x 520 tokens at 128 11.2 -> 13.5, 5 heads
+// 11.5 -> 12.9, but at 768 14.4 -> 14.1 and 14.8 -> 13.5.
 constexpr int64_t kMinSavedElements = int64_t(1) << 23;
+constexpr int64_t kMinCutDenseTokens = 768;
 
 int head_groups(int group, int hg) { return (group + hg - 1) / hg; }
 int even_hg(int group) { return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }
-int pick_hg(int group, int64_t kv_units, int64_t seq_len, int head_dim) {
+bool packed_rows(int fmt) { return fmt == 2 || fmt == 3 || fmt == 4; }
+int pick_hg(int group, int64_t kv_units, int64_t seq_len, int fmt, int head_dim) {
   const int hg = even_hg(group);
-  if (hg == 4 || group < 3) return hg;
+  if (hg == 4 || group < 3 || (!packed_rows(fmt) && seq_len < kMinCutDenseTokens)) return hg;
   const int64_t saved = kv_units * (head_groups(group, hg) - head_groups(group, 4)) * seq_len * head_dim;
   return saved >= kMinSavedElements ? 4 : hg;
 }
@@ -1643,10 +1648,11 @@ constexpr int kMergeWork = 12;  // the merge launch that more than one split add
 // whose count it changes: 1.03 to 1.41 times as fast.  The overheads keep it
 // from short sequences, where more splits lose (640 units x 2235 tokens at
 // head_dim 256: 65 us at 1 split, 67.5 at 2).
+int64_t plan_work(int units, int64_t ns, int64_t blocks, int num_cus) {
+  return ((units * ns + num_cus - 1) / num_cus) * (kLoadOverhead + (blocks + ns - 1) / ns) + (ns > 1 ? kMergeWork : 0);
+}
 int balanced_splits(int units, int ns0, int64_t blocks, int num_cus) {
-  auto work = [&](int64_t ns) {
-    return ((units * ns + num_cus - 1) / num_cus) * (kLoadOverhead + (blocks + ns - 1) / ns) + (ns > 1 ? kMergeWork : 0);
-  };
+  auto work = [&](int64_t ns) { return plan_work(units, ns, blocks, num_cus); };
   int best = ns0;
   const int64_t most = std::min<int64_t>({static_cast<int64_t>(kMaxLoad) * num_cus / units, blocks, kMaxSplits});
   for (int64_t ns = ns0 + 1; ns <= most; ++ns)
@@ -1757,7 +1763,7 @@ int device_scratch(hipStream_t stream, void** out) {
 // per wavefront (64 / (D / slice dims)) x wavefronts; packed slices hold 16
 // dimensions, fp16 rows 8, fp32 rows 4.
 int decode_block_rows(int fmt, int head_dim, int tokens_per_iter = kTokensPerIter) {
-  const bool packed = fmt == 2 || fmt == 3 || fmt == 4;
+  const bool packed = packed_rows(fmt);
   const int slice_dims = packed ? 16 : (fmt == 16 ? 8 : 4);
   return tokens_per_iter * kWavesPerBlock * kWave * slice_dims / head_dim;
 }
@@ -1824,7 +1830,7 @@ constexpr int kShortTokens = 512;
 constexpr int kShortIterations = 8;
 
 bool one_split(int64_t seq_len, int fmt, int head_dim, int hg, int64_t units, int num_cus, bool one_launch) {
-  if (fmt != 2 && fmt != 3 && fmt != 4) return false;
+  if (!packed_rows(fmt)) return false;
   int iterations = kShortIterations;
   if (!one_launch && 2 * units <= num_cus) iterations = (head_dim == 256 ? 8 : 6) - (hg > 1);
   return seq_len <= std::min(kShortTokens, iterations * decode_block_rows(fmt, head_dim));
@@ -1854,7 +1860,7 @@ struct KernelChoice {
 KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int fmt, int head_dim, int group, int flags,
                            int num_cus) {
   if (num_cus <= 0) num_cus = 256;
-  int hg = pick_hg(group, kv_units, seq_len, head_dim);
+  int hg = pick_hg(group, kv_units, seq_len, fmt, head_dim);
   // Units of 4 cost a workgroup of an odd group more than the rows they save
   // where an explicit count leaves every unit of 1 a CU of its own: 4 KV heads
   // x 30000 3-bit tokens at head_dim 64, groups of 7, 8 splits (224 workgroups)
@@ -1899,14 +1905,25 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
     if (runs) return {SplitKernel::Mx, ns, hg};
   }
   if (n_splits > 0) return {SplitKernel::Fp32, n_splits, hg};
-  const int ns0 = default_splits(units, seq_len, num_cus, 2);
   // one split per kMinTokensPerSplit tokens at most, as in default_splits
   const int64_t by_len = (seq_len + kMinTokensPerSplit - 1) / kMinTokensPerSplit;
-  if (ns0 >= by_len) return {SplitKernel::Fp32, ns0, hg};
-  const bool packed = fmt == 2 || fmt == 3 || fmt == 4;
-  const int64_t rows = decode_block_rows(packed ? fmt : 16, head_dim);  // dense rows: one plan for both types
-  const int ns = balanced_splits(units, ns0, (seq_len + rows - 1) / rows, num_cus);
-  return {SplitKernel::Fp32, static_cast<int>(std::min<int64_t>(ns, by_len)), hg};
+  const int64_t rows = decode_block_rows(packed_rows(fmt) ? fmt : 16, head_dim);  // dense rows: one plan for both types
+  const int64_t fp32_blocks = (seq_len + rows - 1) / rows;
+  int ns0 = default_splits(units, seq_len, num_cus, 2);
+  if (ns0 < by_len)
+    ns0 = static_cast<int>(std::min<int64_t>(balanced_splits(units, ns0, fp32_blocks, num_cus), by_len));
+  // Groups cut into units of 4: where the units that divide the group fill the
+  // CUs with one split each, the splits that fewer units take have to pay for
+  // a merge of their own.  Below 2/3 of the work one split is the faster one:
+  // 96 units x 5 heads, 3-bit rows at head_dim 128, 768 tokens 12.6 us in units
+  // of 1, 16.3 cut with 2 splits, 12.6 cut with one, 1536 tokens 20.2, 22.2 and
+  // 20.5; 128 x 3 heads 768 tokens 12.4, 13.2, 12.5, 1024 15.1, 14.0, 15.2; 64 x 7
+  // heads 4-bit at 64, 768 tokens 9.0, 10.6, 7.9.  Fewer units than a third of
+  // the CUs leave too many of them idle: 64 x 3 heads 768 tokens 11.7, 10.7, 12.6.
+  if (hg > even_hg(group) && 3 * units >= num_cus &&
+      3 * plan_work(units, 1, fp32_blocks, num_cus) <= 2 * plan_work(units, ns0, fp32_blocks, num_cus))
+    ns0 = 1;
+  return {SplitKernel::Fp32, ns0, hg};
 }
 
 // Fills the split plan of a decode call over `fmt` rows (see
@@ -1921,7 +1938,7 @@ int make_plan(int num_layers, int kv_heads, int query_heads, int64_t seq_len, in
   if (seq_len < 0) return fail(TQ_ERR_BAD_ARG, "seq_len must be non-negative");
   const int group = query_heads / kv_heads;
   const int64_t kv_units = static_cast<int64_t>(num_layers) * kv_heads;
-  p->hg = pick_hg(group, kv_units, seq_len, head_dim);
+  p->hg = pick_hg(group, kv_units, seq_len, fmt, head_dim);
   p->n_hgroups = head_groups(group, p->hg);
   // One launch holds at most 2^32 - 1 work-items: units x splits workgroups.
   const int64_t max_wg = ((int64_t(1) << 32) - 1) / kBlock;
