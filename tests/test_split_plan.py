@@ -140,3 +140,12 @@ def test_cut_groups_take_splits_that_pay_for_their_merge(units, group, dim, bits
     if bits:
         name = _lib.split_kernel(1, group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=units, n_splits=0, num_cus=CUS)
         assert name == f"decode_kernel<PackedB{bits},{dim},{4 if cut else 1}>"
+
+
+@pytest.mark.parametrize("kv,group,dim,bits,seq,expected", [
+    (4, 6, 128, 3, 65536, {1: 4, 21: 4, 22: 4, 33: 2, 42: 2, 43: 4}),  # 12 and 8 units: 33 to 42 are two rounds of either
+    (8, 10, 64, 2, 32768, {6: 4, 11: 2, 12: 2, 13: 4}),
+])
+def test_explicit_counts_that_save_no_round_keep_units_of_two(kv, group, dim, bits, seq, expected):
+    heads = lambda n: _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, n_splits=n, num_cus=CUS).rstrip(">").split(",")[2]
+    assert {n: int(heads(n)) for n in expected} == expected

@@ -1861,14 +1861,21 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
                            int num_cus) {
   if (num_cus <= 0) num_cus = 256;
   int hg = pick_hg(group, kv_units, seq_len, fmt, head_dim);
-  // Units of 4 cost a workgroup of an odd group more than the rows they save
-  // where an explicit count leaves every unit of 1 a CU of its own: 4 KV heads
-  // x 30000 3-bit tokens at head_dim 64, groups of 7, 8 splits (224 workgroups)
+  // An explicit count with which units of 4 save no round of workgroups over
+  // the CUs only makes each workgroup longer.  Of an odd group: 4 KV heads x
+  // 30000 3-bit tokens at head_dim 64, groups of 7, 8 splits (224 workgroups)
   // 22.9 us in units of 1, 26.4 in units of 4, 11 splits (308) 20.7 and 21.2,
   // 23 (644) 15.9 and 13.7; 8 x 32768 at 128, groups of 3, 9 splits (216) 34.7
-  // and 39.1, 11 (264) 40.3 and 33.5.  Units of 2 lose to units of 4 from 48
-  // workgroups on.
-  if (n_splits > 0 && even_hg(group) == 1 && kv_units * group * n_splits <= num_cus) hg = 1;
+  // and 39.1, 11 (264) 40.3 and 33.5.  Of dense rows: 8 x 52384 at 128, groups
+  // of 6, 1 split (24) 647 in units of 2 and 710, 10 x 13139, 3 splits (240)
+  // 62.5 and 67.5.  Packed rows in units of 2 lose to units of 4 within one
+  // round (24 workgroups 120.7 and 111.0, 240 41.6 and 38.5), but not within
+  // two (480, 64 rows: 27.5 and 29.3).
+  if (n_splits > 0 && hg > even_hg(group)) {
+    const int own = even_hg(group);
+    auto rounds = [&](int h) { return (kv_units * head_groups(group, h) * n_splits + num_cus - 1) / num_cus; };
+    if (rounds(own) == rounds(hg) && (own == 1 || !packed_rows(fmt) || rounds(own) > 1)) hg = own;
+  }
   const int units = static_cast<int>(kv_units * head_groups(group, hg));
   const bool forced = (flags & TQ_MATRIX_PRODUCTS) != 0;
   const bool takes_mx = mx_shape(fmt, head_dim, group) && (flags & TQ_F32_PRODUCTS) == 0;
