@@ -149,3 +149,13 @@ def test_cut_groups_take_splits_that_pay_for_their_merge(units, group, dim, bits
 def test_explicit_counts_that_save_no_round_keep_units_of_two(kv, group, dim, bits, seq, expected):
     heads = lambda n: _lib.split_kernel(kv, kv * group, dim, bits, 0, _lib.TQ_F16, seq, n_splits=n, num_cus=CUS).rstrip(">").split(",")[2]
     assert {n: int(heads(n)) for n in expected} == expected
+
+
+@pytest.mark.parametrize("units,group,dim,bits,seq,most", [
+    (384, 4, 256, 3, 2048, 1), (384, 4, 256, 3, 3072, 2), (640, 4, 256, 3, 3072, 1), (300, 4, 256, 3, 1536, 1),
+    (384, 1, 256, 3, 1536, 2),  # one head at a time has half the set-up
+    (384, 4, 256, 0, 768, 1), (384, 2, 256, 0, 2048, 1), (192, 8, 256, 0, 1331, 1), (320, 4, 128, 0, 1331, 1),
+    (300, 1, 256, 0, 3072, 5), (192, 4, 128, 0, 2048, 2),
+])
+def test_balanced_counts_leave_plans_that_more_splits_slow_down(units, group, dim, bits, seq, most):
+    assert _splits(units, 1, group, dim, bits, 0, seq) == most

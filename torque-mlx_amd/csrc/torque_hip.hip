@@ -1630,9 +1630,10 @@ constexpr int kMinTokensPerSplit = 128;
 
 // Most workgroups per CU of a plan whose workgroups do not all run at once
 // (see balanced_splits), and the work of a workgroup besides its blocks, in
-// blocks.
+// blocks: 4 heads at head_dim 256 take twice the set-up and combine for half
+// the rows of a block.
 constexpr int kMaxLoad = 6;
-constexpr int kLoadOverhead = 5;
+int load_overhead(int head_dim, int hg) { return head_dim == 256 && hg == 4 ? 12 : 5; }
 constexpr int kMergeWork = 12;  // the merge launch that more than one split adds
 
 // Splits of a call with many units.  One resident round of workgroups leaves
@@ -1641,22 +1642,30 @@ constexpr int kMergeWork = 12;  // the merge launch that more than one split add
 // through its workgroups at the same rate whether one or two are resident, so
 // what counts is the work of the CU with the most.  Starting from the
 // one-round count ns0, take the count that makes it smallest, if that is at
-// least 1/16 less.  Measured on MI355X, 24 layers x 8 KV heads: 3-bit rows at
+// least 1/16 less (1/4 for dense rows, whose one-round plans read memory at
+// 5.5 to 6.3 TB/s already).  Measured on MI355X, 24 layers x 8 KV heads: 3-bit rows at
 // head_dim 128 x 8192 tokens, groups of 4, 74 us at 2 splits, 60 at 4 (768
 // workgroups, 3 to a CU), 64 at 5, 63 at 8; 4-bit rows, groups of 1, 57, 45,
 // 47, 44; at head_dim 64, groups of 2, 36, 30, 31, 31.  Over 24 random shapes
 // whose count it changes: 1.03 to 1.41 times as fast.  The overheads keep it
-// from short sequences, where more splits lose (640 units x 2235 tokens at
-// head_dim 256: 65 us at 1 split, 67.5 at 2).
-int64_t plan_work(int units, int64_t ns, int64_t blocks, int num_cus) {
-  return ((units * ns + num_cus - 1) / num_cus) * (kLoadOverhead + (blocks + ns - 1) / ns) + (ns > 1 ? kMergeWork : 0);
-}
-int balanced_splits(int units, int ns0, int64_t blocks, int num_cus) {
-  auto work = [&](int64_t ns) { return plan_work(units, ns, blocks, num_cus); };
+// from short sequences, where more splits lose (3-bit rows at head_dim 256,
+// groups of 4: 384 units x 1536 tokens 53 us at 1 split, 62 at 2, 640 x 3072
+// 143 and 161).  Dense rows at 256, groups of 4: 384 units x 768 tokens 51 and
+// 69, x 2048 129 and 148; 300 x 3072 172 at 1, 167 at 3, groups of 1 172 and 145 at 5.
+struct Work {
+  int units;
+  int64_t blocks;  // of one sequence
+  int overhead, num_cus;
+  int64_t of(int64_t ns) const {
+    return ((units * ns + num_cus - 1) / num_cus) * (overhead + (blocks + ns - 1) / ns) + (ns > 1 ? kMergeWork : 0);
+  }
+};
+int balanced_splits(const Work& work, int ns0, bool packed) {
+  const int64_t limit = (packed ? 15 : 12) * work.of(ns0);
   int best = ns0;
-  const int64_t most = std::min<int64_t>({static_cast<int64_t>(kMaxLoad) * num_cus / units, blocks, kMaxSplits});
+  const int64_t most = std::min<int64_t>({static_cast<int64_t>(kMaxLoad) * work.num_cus / work.units, work.blocks, kMaxSplits});
   for (int64_t ns = ns0 + 1; ns <= most; ++ns)
-    if (16 * work(ns) <= 15 * work(ns0) && work(ns) < work(best)) best = static_cast<int>(ns);
+    if (16 * work.of(ns) <= limit && work.of(ns) < work.of(best)) best = static_cast<int>(ns);
   return best;
 }
 
@@ -1914,11 +1923,11 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
   if (n_splits > 0) return {SplitKernel::Fp32, n_splits, hg};
   // one split per kMinTokensPerSplit tokens at most, as in default_splits
   const int64_t by_len = (seq_len + kMinTokensPerSplit - 1) / kMinTokensPerSplit;
-  const int64_t rows = decode_block_rows(packed_rows(fmt) ? fmt : 16, head_dim);  // dense rows: one plan for both types
-  const int64_t fp32_blocks = (seq_len + rows - 1) / rows;
+  const bool packed = packed_rows(fmt);
+  const int64_t rows = decode_block_rows(packed ? fmt : 16, head_dim);  // dense rows: one plan for both types
+  const Work work{units, (seq_len + rows - 1) / rows, load_overhead(head_dim, hg), num_cus};
   int ns0 = default_splits(units, seq_len, num_cus, 2);
-  if (ns0 < by_len)
-    ns0 = static_cast<int>(std::min<int64_t>(balanced_splits(units, ns0, fp32_blocks, num_cus), by_len));
+  if (ns0 < by_len) ns0 = static_cast<int>(std::min<int64_t>(balanced_splits(work, ns0, packed), by_len));
   // Groups cut into units of 4: where the units that divide the group fill the
   // CUs with one split each, the splits that fewer units take have to pay for
   // a merge of their own.  Below 2/3 of the work one split is the faster one:
@@ -1927,9 +1936,7 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
   // 20.5; 128 x 3 heads 768 tokens 12.4, 13.2, 12.5, 1024 15.1, 14.0, 15.2; 64 x 7
   // heads 4-bit at 64, 768 tokens 9.0, 10.6, 7.9.  Fewer units than a third of
   // the CUs leave too many of them idle: 64 x 3 heads 768 tokens 11.7, 10.7, 12.6.
-  if (hg > even_hg(group) && 3 * units >= num_cus &&
-      3 * plan_work(units, 1, fp32_blocks, num_cus) <= 2 * plan_work(units, ns0, fp32_blocks, num_cus))
-    ns0 = 1;
+  if (hg > even_hg(group) && 3 * units >= num_cus && 3 * work.of(1) <= 2 * work.of(ns0)) ns0 = 1;
   return {SplitKernel::Fp32, ns0, hg};
 }
 
