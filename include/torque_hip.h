@@ -147,8 +147,8 @@ int tq_unpack_dequantize_scaled(const uint32_t* codes, const float* scales, int6
 /* Split count a decode call over `bits`-bit rows (0 for dense rows) with
  * decode `flags` uses when n_splits <= 0 is passed, on num_cus compute units
  * (<= 0: the current device's).  Passed explicitly, this count runs the same
- * split kernel, except that a short sequence's count of 1 may run the matrix
- * kernel where the default runs the float32 kernel.  The sequence is dealt out
+ * split kernel, except that a count of 1 may run the matrix kernel, or units of
+ * fewer query heads, where the default runs the float32 kernel in units of 4.  The sequence is dealt out
  * to the splits in blocks of one workgroup iteration (split s takes blocks s,
  * s + n, s + 2n, ...); an explicit n_splits above the number of blocks is
  * lowered to it. */

@@ -159,3 +159,12 @@ def test_explicit_counts_that_save_no_round_keep_units_of_two(kv, group, dim, bi
 ])
 def test_balanced_counts_leave_plans_that_more_splits_slow_down(units, group, dim, bits, seq, most):
     assert _splits(units, 1, group, dim, bits, 0, seq) == most
+
+
+@pytest.mark.parametrize("units,group,dim,bits,seq,expected", [
+    (160, 6, 128, 4, 1311, 2), (96, 10, 64, 2, 1317, 2), (160, 6, 128, 4, 12000, 4), (176, 6, 128, 4, 1311, 4),
+])
+def test_one_split_of_two_rounds_keeps_units_of_two(units, group, dim, bits, seq, expected):
+    """480 units of 2 and 320 (288) units of 4 are two rounds of workgroups either way; 528 are three."""
+    name = lambda n: _lib.split_kernel(1, group, dim, bits, 0, _lib.TQ_F16, seq, num_layers=units, n_splits=n, num_cus=CUS)
+    assert name(0) == name(_splits(units, 1, group, dim, bits, 0, seq)) == f"decode_kernel<PackedB{bits},{dim},{expected}>"

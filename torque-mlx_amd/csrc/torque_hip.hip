@@ -1879,11 +1879,15 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
   // of 6, 1 split (24) 647 in units of 2 and 710, 10 x 13139, 3 splits (240)
   // 62.5 and 67.5.  Packed rows in units of 2 lose to units of 4 within one
   // round (24 workgroups 120.7 and 111.0, 240 41.6 and 38.5), but not within
-  // two (480, 64 rows: 27.5 and 29.3).
+  // two (480, 8197 rows at 64: 27.5 and 29.3).  Dense splits shorter than the
+  // default's shortest are set-up for the most part: 64 x 1558 at 128, groups
+  // of 6, 48 splits 38.3 in units of 2 and 42.0.
   if (n_splits > 0 && hg > even_hg(group)) {
     const int own = even_hg(group);
     auto rounds = [&](int h) { return (kv_units * head_groups(group, h) * n_splits + num_cus - 1) / num_cus; };
-    if (rounds(own) == rounds(hg) && (own == 1 || !packed_rows(fmt) || rounds(own) > 1)) hg = own;
+    const bool dense = !packed_rows(fmt);
+    if (rounds(own) == rounds(hg) && (own == 1 || dense || rounds(own) > 1)) hg = own;
+    if (dense && own > 1 && seq_len < static_cast<int64_t>(n_splits) * kMinTokensPerSplit) hg = own;
   }
   const int units = static_cast<int>(kv_units * head_groups(group, hg));
   const bool forced = (flags & TQ_MATRIX_PRODUCTS) != 0;
@@ -1936,7 +1940,11 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
   // 20.5; 128 x 3 heads 768 tokens 12.4, 13.2, 12.5, 1024 15.1, 14.0, 15.2; 64 x 7
   // heads 4-bit at 64, 768 tokens 9.0, 10.6, 7.9.  Fewer units than a third of
   // the CUs leave too many of them idle: 64 x 3 heads 768 tokens 11.7, 10.7, 12.6.
-  if (hg > even_hg(group) && 3 * units >= num_cus && 3 * work.of(1) <= 2 * work.of(ns0)) ns0 = 1;
+  const int own = even_hg(group);
+  if (hg > own && 3 * units >= num_cus && 3 * work.of(1) <= 2 * work.of(ns0)) ns0 = 1;
+  // As with explicit counts: 160 x 6 heads, 1311 4-bit scaled tokens at 128 24.8
+  // us in one split of 480 units of 2, 25.9 in one of 320 units of 4.
+  if (hg > own && ns0 == 1 && units > num_cus && kv_units * head_groups(group, own) <= 2 * num_cus) hg = own;
   return {SplitKernel::Fp32, ns0, hg};
 }
 
