@@ -1,13 +1,13 @@
 """The append kernel at its edges: packed words bit for bit against the oracle.
 
-Row counts around the line between the two kernels (4096 rows of both streams), around a workgroup's rows (64, 32, 16
+Row counts around the line between the two kernels (4096 to 8192 rows of both streams when packing), around a workgroup's rows (64, 32, 16
 at head_dim 64, 128, 256) and groups that end inside a wavefront,
 sources that are not 16-byte aligned, quotients that tie with a boundary, values without an ordinary quotient (zeros,
 subnormals, infinities, NaN), and codebooks that the bucket lookup cannot take (equal, unordered, infinite boundaries).
 Whole-number outputs: no tolerance.
 
-The forms with per-vector scales and those that write centroid values run here above the line, where the other tests of
-those entry points stay below it: bit for bit the same as calls of few rows, codes and centroids against the oracle on
+The forms with per-vector scales and those that write centroid values run here on both sides of their lines, where the
+other tests of those entry points stay below them: bit for bit the same as calls of few rows, codes and centroids against the oracle on
 the kernel's own scales.
 """
 
@@ -71,7 +71,7 @@ def _check(x, signs, boundaries, bits, **kwargs):
 @pytest.mark.parametrize("groups,seq_new,dtype,shift", [
     (1, 1, np.float16, 0), (3, 1, np.float32, 0), (1, 15, np.float16, 0), (5, 7, np.float32, 1), (1, 65, np.float16, 3),
     (2, 64, np.float32, 0), (7, 33, np.float16, 0), (3, 1367, np.float32, 0), (2048, 1, np.float16, 0), (5, 411, np.float16, 1),
-    (1, 4111, np.float32, 1), (300, 7, np.float16, 0),
+    (1, 4111, np.float32, 1), (300, 7, np.float16, 0), (5, 823, np.float16, 1), (600, 7, np.float32, 0),
 ])
 def test_row_counts_and_alignment(hip_device, bits, head_dim, groups, seq_new, dtype, shift):
     rng = np.random.default_rng(bits * 1000 + head_dim + seq_new)
@@ -106,7 +106,7 @@ def test_ties_and_special_values(hip_device, head_dim, rotate):
         mixed[0, :], mixed[1, 3], mixed[2, 5], mixed[3, :] = 0.0, np.inf, np.nan, 2e38
         mixed[4] *= 1e-40
         x = np.concatenate([x, mixed])
-        for rows in (x, np.resize(x, (2100, head_dim))):  # a wavefront per row, then 16 elements to a lane
+        for rows in (x, np.resize(x, (2100, head_dim)), np.resize(x, (4200, head_dim))):  # a wavefront per row, then 16 elements to a lane
             _check(rows, signs, bnd, bits, seq_new=rows.shape[0], rotate=rotate)
 
 
@@ -114,7 +114,7 @@ def test_ties_and_special_values(hip_device, head_dim, rotate):
 def test_codebooks_without_buckets(hip_device, bits):
     head_dim, n = 128, (1 << bits) - 1
     rng = np.random.default_rng(bits)
-    x = rng.normal(size=(2100, head_dim)).astype(np.float32)
+    x = rng.normal(size=(4200, head_dim)).astype(np.float32)
     signs = o.rotation_signs_from_seed(head_dim, 2)
     close = np.linspace(-1e-3, 1e-3, n)
     close[-1] = 4.0  # all but one share a bucket
@@ -129,10 +129,10 @@ def test_codebooks_without_buckets(hip_device, bits):
 def test_signs_of_any_size(hip_device, head_dim):
     """Sign vectors that are not +-1 take the division per element."""
     rng = np.random.default_rng(head_dim)
-    x = rng.normal(size=(2100, head_dim)).astype(np.float32)
+    x = rng.normal(size=(4200, head_dim)).astype(np.float32)
     signs = [(s * rng.uniform(0.5, 2.0, size=head_dim)).astype(np.float32) for s in o.rotation_signs_from_seed(head_dim, 4)]
     bnd = o.codebook_boundaries(o.build_gaussian_codebook(4, sample_size=5000, seed=1))
-    _check(x, signs, bnd, 4, seq_new=2100)
+    _check(x, signs, bnd, 4, seq_new=4200)
 
 
 def _stream():
@@ -158,6 +158,14 @@ def _sources(rows, head_dim, dtype, shift, seed):
     return out
 
 
+def _unpack(words, bits, head_dim):
+    """Codes of packed rows: element e at bit e * bits of the row."""
+    at = torch.arange(head_dim, device=words.device) * bits
+    wide = words.to(torch.int64) & 0xFFFFFFFF
+    pair = wide | torch.nn.functional.pad(wide, (0, 1))[:, 1:] << 32  # bits up to 31 of the next word: the last row word has none
+    return (pair[:, at // 32] >> (at % 32)) & ((1 << bits) - 1)
+
+
 def _type(x):
     import torque_hip as th
 
@@ -165,6 +173,7 @@ def _type(x):
 
 
 FORMS = [(2053, torch.float16, 0, 3), (2053, torch.float32, 1, 3), (4500, torch.float32, 0, 3), (4500, torch.float16, 3, 0), (9001, torch.float16, 0, 1)]
+LINES = {4: 16000, 3: 60000, 2: 165000}  # rows of two streams past the largest line of the bit width, when writing values
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
@@ -207,10 +216,11 @@ def test_scaled_rows(hip_device, bits, head_dim, rows, dtype, shift, flags):
 @pytest.mark.parametrize("scaled", [False, True])
 @pytest.mark.parametrize("bits", [2, 3, 4])
 @pytest.mark.parametrize("head_dim", DIMS)
-@pytest.mark.parametrize("rows,dtype,shift,flags", FORMS)
+@pytest.mark.parametrize("rows,dtype,shift,flags", [(2053, torch.float16, 1, 3), (None, torch.float32, 0, 3), (None, torch.float16, 1, 1)])
 def test_dequantized_rows(hip_device, bits, head_dim, rows, dtype, shift, flags, scaled):
     import torque_hip as th
 
+    rows = rows or LINES[bits] // 2 + 37
     keys, values = _sources(rows, head_dim, dtype, shift, bits + head_dim)
     left, right = (torch.from_numpy(s).cuda() for s in o.rotation_signs_from_seed(head_dim, 6))
     kb, kc, vb, vc = _codebooks(bits)
@@ -238,7 +248,7 @@ def test_dequantized_rows(hip_device, bits, head_dim, rows, dtype, shift, flags,
     th._lib.call("tq_append" + name, keys.data_ptr(), values.data_ptr(), _type(keys), 1, 1, rows, head_dim, bits, left.data_ptr(),
                  right.data_ptr(), flags, kb.data_ptr(), vb.data_ptr(), codes[0].data_ptr(), codes[1].data_ptr(), *extra, rows, 0, _stream())
     for i, cent in enumerate((kc, vc)):
-        index = torch.from_numpy(o.unpack_indices_batched(codes[i].cpu().numpy().view(np.uint32), bits, head_dim).astype(np.int64)).cuda()
+        index = _unpack(codes[i], bits, head_dim)
         want = cent[index] * scales[i][:, None] if scaled else cent[index]
         for y in (got[i], few[i], moved[i]):
             assert torch.equal(y.view(torch.int32), want.view(torch.int32))

@@ -178,9 +178,27 @@ __device__ __forceinline__ void pair_step(float (&v)[16], float pair) {
 }
 
 constexpr int kAppendBuckets = 64;
-// Rows (of both streams) up to which append_few_kernel runs: 16 wavefronts to
-// a CU, all resident at once.
-constexpr int64_t kAppendFewRows = 4096;
+// Rows (of all streams) up to which append_few_kernel runs: append_kernel's
+// tables cost 1.5 to 3 us, its rows less than half.  The lines lie where the
+// two cross on MI355X (us, append_few_kernel / append_kernel, rows of two
+// streams each).  Packing: head_dim 64, 4-bit 3000 rows 4.3 / 4.4, 4096 4.6 /
+// 4.5, 2-bit 3500 4.6 / 4.8, 4096 5.0 / 4.6; 128, 4-bit 2049 4.1 / 4.7, 3000 4.7 /
+// 4.8, scaled 2049 4.7 / 4.9; 256, 4-bit 2049 4.8 / 4.8, 2-bit 3000 4.9 / 5.4, 4096
+// 5.7 / 5.5.  Writing centroid values: 64, 4-bit 6000 5.0 / 5.5, 8000 5.9 / 5.8,
+// 2-bit 34000 12.3 / 13.4; 128, 4-bit 4000 5.7 / 6.3, 3-bit 18000 12.2 / 13.4, 2-bit
+// 34000 18.2 / 21.6; 256, 4-bit 2049 5.5 / 6.0, 3-bit 24000 21.3 / 24.8, 2-bit 70000
+// 61.2 / 63.7, scaled 24000 21.7 / 24.3.
+template <int D, int BITS, bool DEQUANT, bool SCALED>
+constexpr int64_t append_few_rows() {
+  if (!DEQUANT) {
+    if (SCALED || BITS == 3) return (SCALED ? BITS == 4 && D < 256 : D == 64) ? 4608 : 4096;
+    return D == 64 ? 7168 : D == 128 ? 6144 : BITS == 2 ? 8192 : 4096;
+  }
+  if (BITS == 4) return D == 256 ? 5120 : SCALED ? 8192 : 12288;
+  if (BITS == 3) return SCALED ? (D == 256 ? 8192 : 12288) : D == 64 ? 20480 : D == 128 ? 40960 : 57344;
+  if (SCALED) return D == 256 ? 57344 : 20480;
+  return D == 64 ? 81920 : D == 128 ? 98304 : 163840;
+}
 constexpr int kAppendMaxBlocks = 2048;  // 8 wavefronts per SIMD on 256 CUs: one resident wave of workgroups
 
 // Rotate -> quantize -> pack (or dequantize) rows of one stream (grid y: keys,
@@ -461,7 +479,7 @@ __global__ __launch_bounds__(kBlock) void append_kernel(const AppendArgs a) {
   }
 }
 
-// The same for a few rows (kAppendFewRows): one wavefront per row, D / 64
+// The same for a few rows (append_few_rows): one wavefront per row, D / 64
 // elements to a lane, codes counted one boundary at a time and packed through
 // LDS.  It has no tables to set up: one token x 4 heads at head_dim 256 takes
 // 2.9 us against append_kernel's 4.3, 64 tokens x 8 heads at 64 3.4 against
@@ -496,9 +514,14 @@ __global__ __launch_bounds__(kBlock) void append_few_kernel(const AppendArgs a) 
     if constexpr (DEQUANT) {
       const float* cent = is_v ? a.value_cent : a.key_cent;
       float* dst = (is_v ? a.value_out : a.key_out) + static_cast<int64_t>(r) * D + lane * E;
+      // every load before the first store, which might alias the tables
 #pragma unroll
-      for (int i = 0; i < E; ++i) dst[i] = SCALED ? cent[quantize_count<BITS>(v[i], bnd)] * scale
-                                                  : cent[quantize_count<BITS>(v[i], bnd)];
+      for (int i = 0; i < E; ++i) {
+        v[i] = cent[quantize_count<BITS>(v[i], bnd)];
+        if (SCALED) v[i] = v[i] * scale;
+      }
+#pragma unroll
+      for (int i = 0; i < E; ++i) dst[i] = v[i];
     } else {
 #pragma unroll
       for (int i = 0; i < E; ++i) s_codes[wave][lane * E + i] = static_cast<uint8_t>(quantize_count<BITS>(v[i], bnd));
@@ -2448,7 +2471,7 @@ int launch_append_part(const AppendParams& p, int64_t g0, int64_t t0, int64_t se
   const uintptr_t bits = reinterpret_cast<uintptr_t>(a.keys) | reinterpret_cast<uintptr_t>(a.values) |
                          reinterpret_cast<uintptr_t>(a.key_out) | reinterpret_cast<uintptr_t>(a.value_out);
   a.wide = bits % 16 == 0;
-  if (rows * p.streams <= kAppendFewRows) {
+  if (rows * p.streams <= append_few_rows<D, BITS, DQ, SC>()) {
     const unsigned few = static_cast<unsigned>((rows + kWavesPerBlock - 1) / kWavesPerBlock);
     hipLaunchKernelGGL((append_few_kernel<D, BITS, T, DQ, SC>), dim3(few, p.streams), dim3(kBlock), 0, stream, a);
     return launch_status("append_few_kernel");
