@@ -131,6 +131,7 @@ def test_units_of_8_take_splits_that_pay_for_their_merge(layers, kv, group, dim,
 @pytest.mark.parametrize("units,group,dim,bits,seq,most,cut", [
     (96, 5, 128, 3, 768, 1, True), (96, 5, 128, 3, 1536, 1, True), (96, 5, 128, 3, 2048, 2, True),
     (128, 3, 128, 3, 768, 1, True), (128, 3, 128, 3, 1024, 4, True), (64, 3, 128, 3, 768, 6, True),  # 64 units: CUs left idle
+    (40, 7, 128, 4, 341, 1, True), (40, 7, 128, 4, 512, 1, True), (36, 7, 128, 4, 400, 3, True),  # 280 and 252 units of 1
     (96, 7, 64, 4, 768, 1, True), (128, 6, 256, 4, 768, 1, True), (128, 5, 128, 3, 600, 1, True),
     (128, 4, 128, 3, 768, 4, True),  # units that divide the group keep their plan
     (64, 7, 128, 0, 767, 1, False), (64, 7, 128, 0, 768, 4, True), (96, 5, 128, 0, 768, 1, True),  # dense rows: cut from 768 tokens on

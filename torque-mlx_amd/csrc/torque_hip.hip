@@ -1854,17 +1854,19 @@ int mx_min_blocks_per_split(int head_dim) { return head_dim == 256 ? 8 : 4; }
 // 7.75; at 256, groups of 1, 256 tokens (8) 7.9 against 8.3, larger units 192
 // tokens (6) 8.0 against 8.5 but 256 9.2 against 9.0.  With more units than
 // half of the CUs the splits do not run side by side and one is faster up to
-// 512 tokens (24 layers x 8 heads, 512 3-bit tokens at 128 9.6 against 15.5).
+// 512 tokens (24 layers x 8 heads, 512 3-bit tokens at 128 9.6 against 15.5);
+// so it is for a group cut into units of 4 whose own units are more than the
+// CUs (40 x 7 heads, 341 4-bit tokens at 128 8.4 in units of 1, 9.3 in 3 splits).
 // A caller whose host pays for the second launch asks for TQ_ONE_LAUNCH: 512
 // tokens x 8 heads at head_dim 128 take 7.6 us on the GPU in one split and 7.1
 // in 4, and 8.6 against 11.6 with the Python call around them.
 constexpr int kShortTokens = 512;
 constexpr int kShortIterations = 8;
 
-bool one_split(int64_t seq_len, int fmt, int head_dim, int hg, int64_t units, int num_cus, bool one_launch) {
+bool one_split(int64_t seq_len, int fmt, int head_dim, int hg, bool many_units, bool one_launch) {
   if (!packed_rows(fmt)) return false;
   int iterations = kShortIterations;
-  if (!one_launch && 2 * units <= num_cus) iterations = (head_dim == 256 ? 8 : 6) - (hg > 1);
+  if (!one_launch && !many_units) iterations = (head_dim == 256 ? 8 : 6) - (hg > 1);
   return seq_len <= std::min(kShortTokens, iterations * decode_block_rows(fmt, head_dim));
 }
 
@@ -1919,7 +1921,8 @@ KernelChoice choose_kernel(int64_t kv_units, int64_t seq_len, int n_splits, int 
   const int min_blocks = mx_min_blocks_per_split(head_dim);
   const int ns4 = default_splits(units, seq_len, num_cus, 1);
   const bool one_launch = forced || (flags & TQ_ONE_LAUNCH) != 0;
-  if (n_splits <= 0 && one_split(seq_len, fmt, head_dim, hg, units, num_cus, one_launch)) {
+  const bool many_units = 2 * units > num_cus || kv_units * head_groups(group, even_hg(group)) > num_cus;
+  if (n_splits <= 0 && one_split(seq_len, fmt, head_dim, hg, many_units, one_launch)) {
     // the matrix kernel where its own plan is one split of enough blocks: 24
     // layers x 8 KV heads x 512 4-bit tokens in groups of 4 at head_dim 128
     // 7.3 us against 9.0, at 64 6.2 against 6.3, 2-bit rows 7.2 against 8.2
